@@ -12,14 +12,29 @@
 // r is byte c of the row, i.e. byte c % 4 (lowest first) of uint32 word
 // w[r * cols/4 + c/4]; value = byte * scale[r, c/64] + bias[r, c/64].
 //
-// Two kernels:
-//   router_logits_kernel  one wave per (expert row, block of NT tokens): lane l
-//       holds bytes 32l .. 32l+31 of each 2048-column piece (two 16-B loads),
-//       converts them with v_cvt_f32_ubyte and accumulates in fp32 in the
-//       factored form; a lane-group sum per token. x stays fp32. All NT
-//       tokens' x loads are issued together and the logits stored at the
-//       end (a store between tokens would hold the next token's loads:
-//       vmcnt counts stores too).
+// Kernels:
+//   router_logits_kernel  one token, or a few bf16 ones, on the vector units:
+//       one wave per (expert row, block of NT tokens); lane l holds bytes
+//       32l .. 32l+31 of each 2048-column piece (two 16-B loads), converts
+//       them with v_cvt_f32_ubyte and accumulates in fp32 in the factored
+//       form; a lane-group sum per token. x stays fp32. All NT tokens' x
+//       loads are issued together and the logits stored at the end (a store
+//       between tokens would hold the next token's loads: vmcnt counts
+//       stores too).
+//   router_logits_mfma_kernel  several tokens, as matrix products: the bytes
+//       become the exact fp16 integers q - 128, x the fp16 pair hi + lo of
+//       x 2^-e with e per (token, group) (22 bits; a bf16 x is exact in hi),
+//       and per group logit += s 2^e P + (b + 128 s) sum(x) in fp32. The
+//       products are exact and a stored scale of ~-128 times the bias no
+//       longer cancels, so the logits are closer to the fp64 product than
+//       the vector form's (1.1e-7 against 2.5e-7 relative). NW waves split K.
+//       What bounded the first form of it, at 25-30 us a block, was the
+//       operand order itself: a lane per matrix row makes a 16-byte load
+//       touch 64 different lines (38 B/ns per CU from L2 against 125-148
+//       where each four lanes read 64 consecutive bytes, measured), so tiles
+//       are read in quads and turned through LDS.
+//   router_logits_block_kernel  many tokens: the same products, 16 tokens by
+//       all experts per workgroup, x converted once, top-8 included.
 //   router_top8_kernel    one wave per token: the logits in registers (up to
 //       4 per lane), eight rounds of a wave maximum (DPP) and a ballot for
 //       the lowest index holding it, then the reference's softmax and
@@ -29,12 +44,6 @@
 #include "mfma.hpp"
 
 namespace qff {
-
-// tokens per logits workgroup: 1 for a single token, else 4 (at batch 16,
-// 4 tokens a wave: logits 7.7-7.8 us event-timed, against 11.3 with 8 and
-// 7.9-8.0 with 2; 12.3 with 8 tokens a wave each waiting for the previous
-// one's store)
-static int rt_tokens(int batch) { return batch <= 1 ? 1 : 4; }
 
 template <int I>
 __device__ __forceinline__ float rt_ubyte(uint32_t v) { return static_cast<float>((v >> (8 * I)) & 0xffu); }
@@ -123,14 +132,213 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint32_t* __re
     }
 }
 
-// grid ceil(batch / 4), 256 threads: wave w ranks token 4 blockIdx.x + w.
-__global__ __launch_bounds__(256) void router_top8_kernel(const float* __restrict__ logits,
-                                                          int32_t* __restrict__ indices, float* __restrict__ scores,
-                                                          int experts, int batch) {
-    const int lane = threadIdx.x & 63;
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (m >= batch) return;   // wave-uniform
-    const float* lg = logits + static_cast<size_t>(m) * experts;
+// Several tokens. grid (ceil(E / (16 NT)), ceil(batch / 16)), NW waves.
+typedef _Float16 rt_f16x2_t __attribute__((ext_vector_type(2)));
+
+// 4 weight bytes -> the fp16 pairs q - 128 (exact): byte b under the exponent
+// byte 0x64 is the fp16 1024 + b, minus 1152
+__device__ __forceinline__ void rt_bytes_to_f16(uint32_t w, uint32_t& lo, uint32_t& hi) {
+    const rt_f16x2_t k = {static_cast<_Float16>(1152.0f), static_cast<_Float16>(1152.0f)};
+    lo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(rt_f16x2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)) - k);
+    hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(rt_f16x2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u)) - k);
+}
+
+// One group (64 columns) of one token, held by the four lanes j of a quad (fp32:
+// columns 16 i + 4 j .. +3 in piece i; bf16: 32 i + 8 j .. +7), as fp16 operands
+// x 2^-e with the group's largest magnitude in [2^13, 2^14) (e >= -127: 2^-e
+// stays finite), hi + lo for fp32 (22 bits; bf16 is exact in hi), into the LDS
+// rows hi, lo [token][row] at 16-byte pieces p0 + c, swizzled by the token.
+// Returns (sum of x, 2^e).
+template <bool HILO, int XL>
+__device__ __forceinline__ float2 rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* hi, uint16_t* lo, int row, int tok,
+                                             int p0, int j) {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < XL; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (HILO) {
+                v[4 * i + c] = __uint_as_float(xr[i][c]);
+            } else {
+                v[8 * i + 2 * c] = __uint_as_float(xr[i][c] << 16);
+                v[8 * i + 2 * c + 1] = __uint_as_float(xr[i][c] & 0xffff0000u);
+            }
+        }
+    float sum = 0.0f, mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        sum += v[i];
+        mx = fmaxf(mx, fabsf(v[i]));
+    }
+    sum = group_sum<4>(sum);
+    mx = group_max<4>(mx);
+    const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 14, -127) : 0;
+    const float p = ldexpf(1.0f, -e);
+    const int sw = tok & (row / 8 - 1) & 15;
+    if (HILO) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            u32x2_t h2, l2;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                uint32_t hh, ll;
+                split_f16x2(v[4 * i + 2 * c] * p, v[4 * i + 2 * c + 1] * p, hh, ll);
+                h2[c] = hh;
+                l2[c] = ll;
+            }
+            const int o = tok * row + 8 * ((p0 + 2 * i + (j >> 1)) ^ sw) + 4 * (j & 1);
+            *reinterpret_cast<u32x2_t*>(hi + o) = h2;
+            *reinterpret_cast<u32x2_t*>(lo + o) = l2;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            u32x4_t h4;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) h4[c] = pack_f16x2(v[8 * i + 2 * c] * p, v[8 * i + 2 * c + 1] * p);
+            *reinterpret_cast<u32x4_t*>(hi + tok * row + 8 * ((p0 + 4 * i + j) ^ sw)) = h4;
+        }
+    }
+    return make_float2(sum, ldexpf(1.0f, e));
+}
+
+// A 16-row x 64-byte tile from the load's lane order (lane l: row l / 4, piece
+// l % 4, so four lanes read 64 consecutive bytes) into the MFMA operand's (lane
+// l: row l % 16, piece l / 16) through 1 KB of the wave's own LDS, the pieces
+// of a row rotated so that 16 lanes meet every bank group.
+__device__ __forceinline__ u32x4_t rt_tile_turn(uint32_t* buf, u32x4_t v, int lane) {
+    const int r = lane >> 2, n = lane & 15;
+    *reinterpret_cast<u32x4_t*>(buf + 4 * (4 * r + ((lane & 3) ^ (r >> 2)))) = v;
+    __builtin_amdgcn_wave_barrier();
+    const u32x4_t o = *reinterpret_cast<const u32x4_t*>(buf + 4 * (4 * n + ((lane >> 4) ^ (n >> 2))));
+    __builtin_amdgcn_wave_barrier();
+    return o;
+}
+
+template <int SB_DT, int X_DT, int NT, int NW>
+__global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint32_t* __restrict__ w,
+                                                                     const uint16_t* __restrict__ scales,
+                                                                     const uint16_t* __restrict__ biases,
+                                                                     const void* __restrict__ x,
+                                                                     float* __restrict__ logits, int experts, int cols,
+                                                                     int batch, int gmagic) {
+    constexpr bool HILO = X_DT == 0;   // fp32 x: hi + lo operands; bf16 x is exact in hi
+    constexpr int RE = 16 * NT;        // experts per workgroup
+    constexpr int XL = HILO ? 4 : 2;   // 16-byte x loads per lane and group
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int n = lane & 15, kb = lane >> 4;
+    const int G = cols / 64;
+    const int E0 = static_cast<int>(blockIdx.x) * RE, M0 = static_cast<int>(blockIdx.y) * 16;
+    // (s, b + 128 s) of the workgroup's experts, [G][RE]; afterwards the waves' partial logits [NW][RE x 16]
+    constexpr int kSb = 64 * (RE + 2) * 2, kPart = NW * RE * 16;
+    __shared__ __attribute__((aligned(16))) float lds[kSb > kPart ? kSb : kPart];
+    // per wave: a weight tile, the group's x (hi, lo) [16 tokens][64] and each token's (sum, 2^e)
+    __shared__ __attribute__((aligned(16))) uint32_t wl[NW][256];
+    __shared__ __attribute__((aligned(16))) uint16_t xl[NW][HILO ? 2 : 1][16 * 64];
+    __shared__ float2 xf[NW][16];
+
+    const char* xrow = static_cast<const char*>(x) +
+                       static_cast<size_t>(min(M0 + (lane >> 2), batch - 1)) * cols * (HILO ? 4 : 2) + 16 * (lane & 3);
+    const uint32_t* wrow[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+        wrow[i] = w + static_cast<size_t>(min(E0 + 16 * i + (lane >> 2), experts - 1)) * (cols / 4) + 4 * (lane & 3);
+
+    u32x4_t xr[2][XL], wr[2][NT];
+    auto fetch = [&](int s, int g) {
+        const char* xp = xrow + 64 * g * (HILO ? 4 : 2);
+#pragma unroll
+        for (int q = 0; q < XL; ++q) xr[s][q] = *reinterpret_cast<const u32x4_t*>(xp + 64 * q);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) wr[s][i] = *reinterpret_cast<const u32x4_t*>(wrow[i] + 16 * g);
+    };
+    // the wave's first two groups and the scales, all requested before any is
+    // used (indices clamped, so every load is issued)
+    fetch(0, min(wave, G - 1));
+    fetch(1, min(wave + NW, G - 1));
+    constexpr int SBT = RE / NW;   // entries per thread at the largest G, 64
+    float sv[SBT], bv[SBT];
+#pragma unroll
+    for (int k = 0; k < SBT; ++k) {
+        const int idx = min(t + 64 * NW * k, RE * G - 1), e = (idx * gmagic) >> 20;
+        const size_t gi = static_cast<size_t>(min(E0 + e, experts - 1)) * G + (idx - e * G);
+        sv[k] = elem<SB_DT>::load(scales, gi);
+        bv[k] = elem<SB_DT>::load(biases, gi);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < SBT; ++k) {
+        const int idx = min(t + 64 * NW * k, RE * G - 1), e = (idx * gmagic) >> 20, g = idx - e * G;
+        *reinterpret_cast<float2*>(&lds[(g * (RE + 2) + e) * 2]) = make_float2(sv[k], fmaf(128.0f, sv[k], bv[k]));
+    }
+    __syncthreads();
+
+    f32x4_t acc[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto step = [&](int s, int g) {
+        const float2 xs = rt_stage_x<HILO>(xr[s], xl[wave][0], xl[wave][HILO ? 1 : 0], 64, lane >> 2, 0, lane & 3);
+        if ((lane & 3) == 0) xf[wave][lane >> 2] = xs;
+        __builtin_amdgcn_wave_barrier();
+        const float2 sf = xf[wave][n];
+        u32x4_t xh[2], xw[2];
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int o = n * 64 + 8 * ((2 * kb + ks) ^ (n & 7));
+            xh[ks] = *reinterpret_cast<const u32x4_t*>(&xl[wave][0][o]);
+            if (HILO) xw[ks] = *reinterpret_cast<const u32x4_t*>(&xl[wave][HILO ? 1 : 0][o]);
+        }
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const u32x4_t wd = rt_tile_turn(wl[wave], wr[s][i], lane);
+            u32x4_t a[2];
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                uint32_t lo, hi;
+                rt_bytes_to_f16(wd[d], lo, hi);
+                a[d >> 1][2 * (d & 1)] = lo;
+                a[d >> 1][2 * (d & 1) + 1] = hi;
+            }
+            f32x4_t P = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            if (HILO) {
+                P = mfma_16x16x32_f16(a[0], xw[0], P);
+                P = mfma_16x16x32_f16(a[1], xw[1], P);
+            }
+            P = mfma_16x16x32_f16(a[0], xh[0], P);
+            P = mfma_16x16x32_f16(a[1], xh[1], P);
+            // experts 16 i + 4 kb .. +3
+            const f32x4_t* sb = reinterpret_cast<const f32x4_t*>(&lds[(g * (RE + 2) + 16 * i + 4 * kb) * 2]);
+            const f32x4_t c0 = sb[0], c1 = sb[1];
+            acc[i][0] = fmaf(c0[0], P[0] * sf.y, fmaf(c0[1], sf.x, acc[i][0]));
+            acc[i][1] = fmaf(c0[2], P[1] * sf.y, fmaf(c0[3], sf.x, acc[i][1]));
+            acc[i][2] = fmaf(c1[0], P[2] * sf.y, fmaf(c1[1], sf.x, acc[i][2]));
+            acc[i][3] = fmaf(c1[2], P[3] * sf.y, fmaf(c1[3], sf.x, acc[i][3]));
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    for (int g = wave; g < G; g += 2 * NW) {   // wave-uniform
+        step(0, g);
+        if (g + 2 * NW < G) fetch(0, g + 2 * NW);
+        if (g + NW < G) step(1, g + NW);
+        if (g + 3 * NW < G) fetch(1, g + 3 * NW);
+    }
+    __syncthreads();   // the scales are consumed; their bytes take the partial sums
+#pragma unroll
+    for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4_t*>(&lds[wave * RE * 16 + (i * 64 + lane) * 4]) = acc[i];
+    __syncthreads();
+    for (int o = t; o < RE * 16; o += 64 * NW) {
+        float v = lds[o];
+#pragma unroll
+        for (int ww = 1; ww < NW; ++ww) v += lds[ww * RE * 16 + o];
+        const int l = (o >> 2) & 63, e = E0 + 16 * (o >> 8) + 4 * (l >> 4) + (o & 3), m = M0 + (l & 15);
+        if (m < batch && e < experts) logits[static_cast<size_t>(m) * experts + e] = v;
+    }
+}
+
+// One wave ranks token m's logits lg[0 .. experts): the eight largest (ties to
+// the lower index) and their renormalised softmax weights.
+__device__ __forceinline__ void router_top8(const float* lg, int32_t* __restrict__ indices,
+                                            float* __restrict__ scores, int m, int experts, int lane) {
     float v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
@@ -188,6 +396,170 @@ __global__ __launch_bounds__(256) void router_top8_kernel(const float* __restric
     }
 }
 
+
+// grid ceil(batch / 4), 256 threads: wave w ranks token 4 blockIdx.x + w.
+__global__ __launch_bounds__(256) void router_top8_kernel(const float* __restrict__ logits,
+                                                          int32_t* __restrict__ indices, float* __restrict__ scores,
+                                                          int experts, int batch) {
+    const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (m >= batch) return;   // wave-uniform
+    router_top8(logits + static_cast<size_t>(m) * experts, indices, scores, m, experts, threadIdx.x & 63);
+}
+
+// Enough tokens for every CU: a workgroup takes 16 tokens and all experts (wave
+// w experts 32 w .. 32 w + 31, two MFMA tiles over all of K) and ranks its
+// tokens itself. Each slab of 512 columns of x is converted once per
+// workgroup (thread quads, rt_stage_x) into LDS; the weights are requested a
+// slab ahead into registers.
+constexpr int kRtSlab = 8;   // groups per slab
+
+template <int SB_DT, int X_DT, int NW>
+__global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
+    const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
+    const void* __restrict__ x, float* __restrict__ logits, int32_t* __restrict__ indices,
+    float* __restrict__ scores, int experts, int cols, int batch) {
+    constexpr bool HILO = X_DT == 0;
+    constexpr int RE = 32 * NW, XL = HILO ? 4 : 2, QT = 8 / NW;   // QT quads (token, group) per thread and slab
+    static_assert(RE == 256, "a workgroup holds every expert");
+    constexpr int XS = 16 * 512;                                  // fp16 values of a slab
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int n = lane & 15, kb = lane >> 4;
+    const int G = cols / 64, NS = (G + kRtSlab - 1) / kRtSlab;
+    const int M0 = static_cast<int>(blockIdx.x) * 16;
+
+    __shared__ __attribute__((aligned(16))) uint16_t xs[2][HILO ? 2 : 1][XS];
+    __shared__ __attribute__((aligned(16))) float sbl[2][kRtSlab * (RE + 2) * 2];
+    __shared__ __attribute__((aligned(16))) uint32_t wl[NW][2][256];   // per wave: a tile's 16 rows x 64 bytes
+    __shared__ float2 xf[2][kRtSlab][16];   // (sum, 2^e) of (group, token)
+
+    // this thread's x quads and scale entries of a slab, and this wave's
+    // weights of it: lane (row n, kb) bytes 16 kb .. +15 of each group
+    u32x4_t xr[QT][XL], wr[kRtSlab][2];
+    float sv[4], bv[4];
+    const uint32_t* wrow[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        wrow[i] = w + static_cast<size_t>(min(32 * wave + 16 * i + (lane >> 2), experts - 1)) * (cols / 4) + 4 * (lane & 3);
+    auto fetch_x = [&](int sl) {
+#pragma unroll
+        for (int k = 0; k < QT; ++k) {
+            const int q = (t >> 2) + 16 * NW * k, tok = q >> 3, g = min(kRtSlab * sl + (q & 7), G - 1);
+            const char* src = static_cast<const char*>(x) +
+                              (static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 64 * g) * (HILO ? 4 : 2) + 16 * (t & 3);
+#pragma unroll
+            for (int i = 0; i < XL; ++i) xr[k][i] = *reinterpret_cast<const u32x4_t*>(src + 64 * i);
+        }
+    };
+    auto fetch_sb = [&](int sl) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int idx = t + 64 * NW * k, e = idx >> 3, g = kRtSlab * sl + (idx & 7);
+            const size_t gi = static_cast<size_t>(min(e, experts - 1)) * G + min(g, G - 1);
+            sv[k] = elem<SB_DT>::load(scales, gi);
+            bv[k] = elem<SB_DT>::load(biases, gi);
+        }
+    };
+    auto fetch_w = [&](int sl, int gl) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            wr[gl][i] = *reinterpret_cast<const u32x4_t*>(wrow[i] + 16 * min(kRtSlab * sl + gl, G - 1));
+    };
+    // the fetched slab into LDS buffer buf (groups past the last get zero scales)
+    auto stage = [&](int sl, int buf) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int idx = t + 64 * NW * k, e = idx >> 3, gl = idx & 7;
+            const bool live = kRtSlab * sl + gl < G;
+            *reinterpret_cast<float2*>(&sbl[buf][(gl * (RE + 2) + e) * 2]) =
+                make_float2(live ? sv[k] : 0.0f, live ? fmaf(128.0f, sv[k], bv[k]) : 0.0f);
+        }
+#pragma unroll
+        for (int k = 0; k < QT; ++k) {
+            const int q = (t >> 2) + 16 * NW * k, tok = q >> 3, gl = q & 7, j = t & 3;
+            const float2 xs2 = rt_stage_x<HILO>(xr[k], xs[buf][0], xs[buf][HILO ? 1 : 0], 512, tok, 8 * gl, j);
+            if (j == 0) xf[buf][gl][tok] = xs2;
+        }
+    };
+
+    fetch_x(0);
+    fetch_sb(0);
+#pragma unroll
+    for (int gl = 0; gl < kRtSlab; ++gl) fetch_w(0, gl);
+    // (a clobber after each slab's requests: otherwise the compiler moves the
+    // loads to the top of the iteration that uses them)
+    asm volatile("" ::: "memory");
+    f32x4_t tot[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int sl = 0; sl < NS; ++sl) {
+        const int buf = sl & 1;
+        f32x4_t acc[2];   // the slab's own sums: shorter fp32 chains
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        stage(sl, buf);
+        __syncthreads();
+        // the next slab (the last again at the end: no branch around loads)
+        const int nx = min(sl + 1, NS - 1);
+        fetch_x(nx);
+        fetch_sb(nx);
+#pragma unroll
+        for (int gl = 0; gl < kRtSlab; ++gl) {
+            const float2 sf = xf[buf][gl][n];
+            u32x4_t xh[2], xl[2];
+#pragma unroll
+            for (int ks = 0; ks < 2; ++ks) {   // columns 16 kb + 8 ks .. +7 of the group
+                const int o = n * 512 + 8 * ((8 * gl + 2 * kb + ks) ^ n);
+                xh[ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][0][o]);
+                if (HILO) xl[ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][HILO ? 1 : 0][o]);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const u32x4_t wd = rt_tile_turn(wl[wave][i], wr[gl][i], lane);
+                u32x4_t a[2];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) {
+                    uint32_t lo, hi;
+                    rt_bytes_to_f16(wd[d], lo, hi);
+                    a[d >> 1][2 * (d & 1)] = lo;
+                    a[d >> 1][2 * (d & 1) + 1] = hi;
+                }
+                f32x4_t P = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                if (HILO) {
+                    P = mfma_16x16x32_f16(a[0], xl[0], P);
+                    P = mfma_16x16x32_f16(a[1], xl[1], P);
+                }
+                P = mfma_16x16x32_f16(a[0], xh[0], P);
+                P = mfma_16x16x32_f16(a[1], xh[1], P);
+                const f32x4_t* sb = reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 32 * wave + 16 * i + 4 * kb) * 2]);
+                const f32x4_t c0 = sb[0], c1 = sb[1];
+                acc[i][0] = fmaf(c0[0], P[0] * sf.y, fmaf(c0[1], sf.x, acc[i][0]));
+                acc[i][1] = fmaf(c0[2], P[1] * sf.y, fmaf(c0[3], sf.x, acc[i][1]));
+                acc[i][2] = fmaf(c1[0], P[2] * sf.y, fmaf(c1[1], sf.x, acc[i][2]));
+                acc[i][3] = fmaf(c1[2], P[3] * sf.y, fmaf(c1[3], sf.x, acc[i][3]));
+            }
+            fetch_w(nx, gl);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) tot[i] += acc[i];
+        asm volatile("" ::: "memory");
+    }
+    // lane: token n, experts 32 wave + 16 i + 4 kb .. +3
+    // every expert of the 16 tokens is here: logits through LDS (the staging
+    // buffers are idle once every wave is past its last slab)
+    __syncthreads();
+    float* lg = reinterpret_cast<float*>(xs);   // [16][RE + 4]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 32 * wave + 16 * i + 4 * kb]) = tot[i];
+    __syncthreads();
+    for (int tok = wave; tok < 16; tok += NW) {
+        const int m = M0 + tok;
+        if (m >= batch) break;
+        for (int e = lane; e < experts; e += 64) logits[static_cast<size_t>(m) * experts + e] = lg[tok * (RE + 4) + e];
+        router_top8(lg + tok * (RE + 4), indices, scores, m, experts, lane);
+    }
+}
+
 // Q8 dequant test hook: one word (4 bytes) per thread -> 4 floats.
 template <int SB_DT>
 __global__ __launch_bounds__(256) void q8_dequant_kernel(const uint32_t* __restrict__ w,
@@ -224,23 +596,60 @@ hipError_t launch_router_top8(qff_ctx* ctx, hipStream_t stream, const uint32_t* 
                               float* logits, int32_t* indices, float* scores, int experts, int cols, int batch) {
     const uint16_t* s = static_cast<const uint16_t*>(scales);
     const uint16_t* b = static_cast<const uint16_t*>(biases);
-    const int nt = rt_tokens(batch);
-    const dim3 grid((experts + 3) / 4, (batch + nt - 1) / nt);
-    const bool k2 = cols > 2048;
+    // The kernel by the number of 16-token blocks nb (batch 8192 / 2000 / 512 /
+    // 16 at 256 x 2048, both launches, fp32 x, us):
+    //   vector units   1840 / 456 / 123 / 11.6 (bf16 x at 16: 9.5)
+    //   MFMA, 1 tile    158 / 46.4 / 17.8 / 11.2 (bf16 x at 16: 10.1)
+    //   MFMA, 2 tiles    92 / 31.8 / 14.5 / 12.4
+    //   MFMA, 4 tiles    77 / 26.4 / 17.7 / 16.6
+    //   whole blocks     61 / 29.3 / 27.7 / 26.4 (33 against 44.5 at 4096)
+    // so the tiles per workgroup grow once the grid covers the chip, and whole
+    // blocks take over where they do so themselves.
+    const int nb = (batch + 15) / 16, cu = ctx->num_cu;
+    const bool k2 = cols > 2048, vec = batch == 1 || (x_dtype == QFF_BF16 && batch <= 16);
+    if (8 * nb > 5 * cu) {
+        ProfScope prof(ctx, stream, "router_logits");
+#define QFF_RB(S, X) \
+    router_logits_block_kernel<S, X, 8><<<nb, 512, 0, stream>>>(w, s, b, x, logits, indices, scores, experts, cols, batch)
+        if (sb_dtype == QFF_BF16) {
+            if (x_dtype == QFF_BF16) QFF_RB(1, 1); else QFF_RB(1, 0);
+        } else {
+            if (x_dtype == QFF_BF16) QFF_RB(2, 1); else QFF_RB(2, 0);
+        }
+#undef QFF_RB
+        return hipGetLastError();
+    }
     {
         ProfScope prof(ctx, stream, "router_logits");
-#define QFF_RL_NT(S, X, K)                                                                                     \
-    if (nt == 1) router_logits_kernel<S, X, K, 1><<<grid, 256, 0, stream>>>(w, s, b, x, logits, experts, cols, batch); \
-    else router_logits_kernel<S, X, K, 4><<<grid, 256, 0, stream>>>(w, s, b, x, logits, experts, cols, batch)
-#define QFF_RL(S, X)                   \
-    if (k2) { QFF_RL_NT(S, X, 2); }     \
-    else { QFF_RL_NT(S, X, 1); }
+        const dim3 vgrid((experts + 3) / 4, (batch + 3) / 4);
+        const int gmagic = (1 << 20) / (cols / 64) + 1;   // idx / G = idx gmagic >> 20 for idx < 4096, G <= 64
+        const auto tiles = [&](int nt) { return (experts + 16 * nt - 1) / (16 * nt); };
+#define QFF_RV(S, X, K, NT) \
+    router_logits_kernel<S, X, K, NT><<<vgrid, 256, 0, stream>>>(w, s, b, x, logits, experts, cols, batch)
+#define QFF_RM(S, X, NT, NW)                                                                              \
+    router_logits_mfma_kernel<S, X, NT, NW><<<dim3(tiles(NT), nb), 64 * NW, 0, stream>>>(w, s, b, x, logits, \
+                                                                                        experts, cols, batch, gmagic)
+#define QFF_RL(S, X)                                            \
+    if (vec) {                                                  \
+        if (batch == 1) {                                       \
+            if (k2) QFF_RV(S, X, 2, 1); else QFF_RV(S, X, 1, 1); \
+        } else {                                                \
+            if (k2) QFF_RV(S, X, 2, 4); else QFF_RV(S, X, 1, 4); \
+        }                                                       \
+    } else if (tiles(1) * nb <= cu) {                           \
+        QFF_RM(S, X, 1, 16);                                    \
+    } else if (tiles(2) * nb <= cu) {                           \
+        QFF_RM(S, X, 2, 8);                                     \
+    } else {                                                    \
+        QFF_RM(S, X, 4, 4);                                     \
+    }
 #define QFF_RL_X(S) \
     if (x_dtype == QFF_BF16) { QFF_RL(S, 1); } else { QFF_RL(S, 0); }
         if (sb_dtype == QFF_BF16) { QFF_RL_X(1); } else { QFF_RL_X(2); }
 #undef QFF_RL_X
 #undef QFF_RL
-#undef QFF_RL_NT
+#undef QFF_RM
+#undef QFF_RV
     }
     ProfScope prof(ctx, stream, "router_top8");
     router_top8_kernel<<<(batch + 3) / 4, 256, 0, stream>>>(logits, indices, scores, experts, batch);

@@ -68,6 +68,41 @@ def test_router_top8(hip, batch, experts, cols, xdt):
             assert np.array_equal(idx[m], O.router_top8(ol)[0])
 
 
+@pytest.mark.parametrize("batch,experts,cols,xdt,sb", [
+    (2, 256, 2048, "f32", "bf16"), (17, 256, 2048, "bf16", "f16"),     # one tile per workgroup, a ragged token block
+    (257, 40, 4096, "f32", "bf16"), (300, 256, 64, "f32", "f16"),      # two tiles; one group of columns
+    (600, 250, 2048, "bf16", "bf16"), (1000, 8, 1088, "f32", "bf16"),  # four tiles; fewer experts than a tile
+    (2577, 256, 2048, "f32", "bf16"), (2600, 100, 576, "bf16", "f16")  # whole blocks; a ragged slab of columns
+])
+def test_router_top8_many_tokens(hip, batch, experts, cols, xdt, sb):
+    """The matrix-core logits at the edges of their tiles, with tokens scaled
+    by 2^-60 .. 2^60 and an all-zero token: every token within 1e-6 of the
+    fp64 product relative to its own sum of |W x| (fp32 sums of exact
+    products: a few 2^-24), the ranking that of the kernel's own logits."""
+    import qff
+    print(f"router_top8 batch={batch} experts={experts} cols={cols} x={xdt} scales={sb}", flush=True)
+    w, s, b = synth.q8_weight(experts, cols, seed=experts + cols + batch, sb_dtype=sb)
+    rng = np.random.default_rng(batch)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    x *= np.exp2(rng.integers(-60, 61, (batch, 1))).astype(np.float32)
+    x[batch // 2] = 0.0
+    if xdt == "bf16":
+        x = O.round_bf16(x)
+    xt = bf16_tensor(O.f32_to_bf16(x)) if xdt == "bf16" else f32_tensor(x)
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=1)
+    idx, sc, lg = qff.router_top8(ctx, *_w_gpu(w, s, b, sb), xt)
+    torch.cuda.synchronize()
+    idx, sc, lg = idx.cpu().numpy(), sc.cpu().numpy(), lg.cpu().numpy()
+    dense = O.q8_dequant(w, s, b, O.F16 if sb == "f16" else O.BF16).astype(np.float64)
+    err = np.abs(lg - x.astype(np.float64) @ dense.T)
+    assert np.all(err <= 1e-6 * (np.abs(x).astype(np.float64) @ np.abs(dense).T))
+    order = np.argsort(-lg, axis=1, kind="stable")[:, :8]
+    assert np.array_equal(idx, order)
+    top = np.take_along_axis(lg, order, 1).astype(np.float64)
+    p = np.exp(top - top[:, :1])
+    assert np.allclose(sc, p / p.sum(1, keepdims=True), atol=1e-6)
+
+
 def test_router_rejects_bad_calls(hip):
     import qff
     from qff._lib import lib
