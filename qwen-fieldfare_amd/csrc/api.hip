@@ -39,7 +39,7 @@ WorkspaceLayout workspace_layout(const qff_ctx_cfg& cfg) {
     L.gqa_qb = take(T * 16 * 256 * sizeof(uint16_t));
     L.gqa_kv16 = take(static_cast<size_t>(cfg.max_ctx) * 512 * sizeof(uint16_t));
     L.gqa_vt = take(static_cast<size_t>((cfg.max_ctx + 63) / 64) * 64 * 512 * sizeof(uint16_t));
-    L.q4_x16 = take(static_cast<size_t>(q4_xs_tokens(cfg)) * 4096 * sizeof(uint16_t));
+    L.q4_x16 = take(static_cast<size_t>((q4_xs_tokens(cfg) + 31) / 32 * 32) * 4096 * sizeof(uint16_t));   // whole 32-token tiles
     L.q4_fm = take(static_cast<size_t>(q4_xs_tokens(cfg)) * sizeof(float));
     L.q4_sk_part = take(static_cast<size_t>(kQ4SkSlots) * 16 * 64 * sizeof(float));
     const size_t TC = (T + 63) / 64 * 64;   // tokens rounded up to whole chunks

@@ -12,10 +12,13 @@
 // 128 + q by OR-ing it into the mantissa of 0x4300 (128.0), so an MFMA over
 // those operands yields P = sum (128 + q) x, and
 //   sum_c W x = s * P + (b - 128 s) * sum(x)       (per group, per row)
-// with sum(x) over the same bf16-rounded x the MFMA saw. Two kernels:
+// with sum(x) over the same bf16-rounded x the MFMA saw. Kernels:
 // q4_gemv_kernel for decode batches (<= 32 tokens), streaming each weight row
-// once with the K dimension split over a workgroup's waves, and
-// q4_gemm_kernel for many tokens (prefill projections), tiled 128 x 128.
+// once with the K dimension split over a workgroup's waves; many tokens
+// (prefill projections) run on fp16 operands, q4_gemm_split_kernel for short
+// batches (K split over a workgroup's waves) and q4_gemm_kernel, tiled 256 x 128.
+#include <algorithm>
+
 #include "common.hpp"
 #include "internal.hpp"
 #include "mfma.hpp"
@@ -124,12 +127,12 @@ __device__ __forceinline__ Q4Part1 q4_part_of(const Q4Parts& parts, int blk) {
 // in-bounds address (the part's weights stand in for the one not needed),
 // and selected: a branch around a load would make the compiler wait for
 // every load in flight at the join.
-__device__ __forceinline__ f32x4_t q4_res4(const Q4Parts& parts, int p, size_t i, bool ok) {
-    const bool has = ok && parts.res[p] != nullptr, bf = parts.ybf16[p] != 0;
-    const u32x2_t* r16 = has && bf ? reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(parts.res[p]) + i)
-                                   : reinterpret_cast<const u32x2_t*>(parts.w[p]);
-    const u32x4_t* r32 = has && !bf ? reinterpret_cast<const u32x4_t*>(static_cast<const float*>(parts.res[p]) + i)
-                                    : reinterpret_cast<const u32x4_t*>(parts.w[p]);
+__device__ __forceinline__ f32x4_t q4_res4(const Q4Part1& P, size_t i, bool ok) {
+    const bool has = ok && P.res != nullptr, bf = P.ybf16 != 0;
+    const u32x2_t* r16 = has && bf ? reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(P.res) + i)
+                                   : reinterpret_cast<const u32x2_t*>(P.w);
+    const u32x4_t* r32 = has && !bf ? reinterpret_cast<const u32x4_t*>(static_cast<const float*>(P.res) + i)
+                                    : reinterpret_cast<const u32x4_t*>(P.w);
     const u32x2_t a = *r16;
     const u32x4_t b = *r32;
     const f32x4_t r = bf ? f32x4_t{__uint_as_float(a[0] << 16), __uint_as_float(a[0] & 0xffff0000u),
@@ -137,6 +140,9 @@ __device__ __forceinline__ f32x4_t q4_res4(const Q4Parts& parts, int p, size_t i
                          : f32x4_t{__uint_as_float(b[0]), __uint_as_float(b[1]), __uint_as_float(b[2]),
                                    __uint_as_float(b[3])};
     return has ? r : f32x4_t{0.f, 0.f, 0.f, 0.f};
+}
+__device__ __forceinline__ f32x4_t q4_res4(const Q4Parts& parts, int p, size_t i, bool ok) {
+    return q4_res4(Q4Part1{parts.w[p], nullptr, nullptr, nullptr, parts.res[p], 0, parts.ybf16[p], 0}, i, ok);
 }
 // y[i] of part p = v, in the part's output dtype
 __device__ __forceinline__ void q4_put(const Q4Parts& parts, int p, size_t i, float v) {
@@ -948,19 +954,34 @@ __global__ __launch_bounds__(64 * kQ4VecWaves) void q4_gemv1_kernel(Q4Parts part
 constexpr int kQ4GemmRows = 256;   // weight rows per workgroup
 constexpr int kQ4GemmToks = 128;   // tokens per workgroup
 
-// x16 and f_m of one token per wave: lane l holds 8-column blocks l, l + 64, ...
-template <int X_DT, bool NORM>
-__global__ __launch_bounds__(256) void q4_x16_kernel(const void* __restrict__ x, uint16_t* __restrict__ x16,
+// x16 lies in the order of the 32x32x16 MFMA's B operand: per token tile of 32,
+// group of 64 columns and step ks a block of 64 lanes x 16 bytes, lane 32 h + r
+// holding token r's 8-column piece 4 h + ks of the group, so an operand is one
+// contiguous 1-KB read (a lane per token row costs the load unit four times
+// as many cycles). `piece` is the token's 8-column block over the row.
+__device__ __forceinline__ size_t q4_x16_at(int m, int piece, int G) {
+    const int g = piece >> 3, h = (piece >> 2) & 1, ks = piece & 3;
+    return ((static_cast<size_t>(m >> 5) * G + g) * 4 + ks) * 512 + (32 * h + (m & 31)) * 8;
+}
+
+// x16 and f_m, WPT waves per token: thread i of a token's 64 WPT holds 8-column
+// blocks i, i + 64 WPT, .. One wave per token (TPB tokens a workgroup) where
+// the tokens fill the chip; four for short batches, whose time is one wave's
+// chain of loads, maxima and stores.
+template <int X_DT, bool NORM, int WPT, int TPB>
+__global__ __launch_bounds__(64 * WPT * TPB) void q4_x16_kernel(const void* __restrict__ x, uint16_t* __restrict__ x16,
                                                      float* __restrict__ fm, int cols, int batch, Q4Norm nrm) {
-    const int m = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-    if (m >= batch) return;
-    const int nb = cols / 8;
-    constexpr int kMaxB = 4096 / 8 / 64;
+    static_assert(WPT == 1 || TPB == 1, "several waves a token, or several tokens a workgroup");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i0 = TPB > 1 ? lane : static_cast<int>(threadIdx.x);
+    const int mt = blockIdx.x * TPB + (TPB > 1 ? wave : 0);   // this wave's token
+    const int m = min(mt, batch - 1);
+    const int nb = cols / 8, G = cols / 64;
+    constexpr int kMaxB = 4096 / 8 / (64 * WPT);
     float v[kMaxB][8];
     float ss = 0.0f, mx = 0.0f;
 #pragma unroll
     for (int i = 0; i < kMaxB; ++i) {
-        const int b = lane + 64 * i;
+        const int b = i0 + 64 * WPT * i;
         if (b < nb) {
             const size_t o = static_cast<size_t>(m) * cols + 8 * b;
             if (X_DT == 1) {
@@ -989,28 +1010,48 @@ __global__ __launch_bounds__(256) void q4_x16_kernel(const void* __restrict__ x,
             for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[i][e]));
         }
     }
+    mx = group_max<64>(mx);
+    if (NORM) ss = group_sum<64>(ss);
+    if constexpr (WPT > 1) {
+        __shared__ float2 part[WPT];
+        if (lane == 0) part[threadIdx.x >> 6] = make_float2(mx, ss);
+        __syncthreads();
+        mx = part[0].x;
+        ss = part[0].y;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+        for (int w = 1; w < WPT; ++w) {
+            mx = fmaxf(mx, part[w].x);
+            ss += part[w].y;
+        }
+    }
     // max |x'| in [2^(E-1), 2^E): x' 2^-(E-14) stays below 2^14. e >= -127
     // keeps 2^-e a finite fp32 for the smallest tokens (fp32 subnormals
     // included): their x16 then sits below 2^14 but stays in fp16's normal
     // range down to |x'| = 2^-141, and f_m >= 2^-135 keeps 14 bits.
     const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 14, -127) : 0;
     const float p = ldexpf(1.0f, -e);
+    // TPB tokens meet in LDS per 64 blocks, so that TPB lanes write 16 TPB
+    // consecutive bytes (a lane per block writes 64 separate lines an
+    // instruction: 14 us more at 8192 x 4096)
+    __shared__ u32x4_t xo[TPB > 1 ? 2 : 1][TPB > 1 ? 64 * (TPB + 1) : 1];
 #pragma unroll
     for (int i = 0; i < kMaxB; ++i) {
-        const int b = lane + 64 * i;
-        if (b < nb) {
-            const u32x4_t h{pack_f16x2(v[i][0] * p, v[i][4] * p), pack_f16x2(v[i][1] * p, v[i][5] * p),
-                            pack_f16x2(v[i][2] * p, v[i][6] * p), pack_f16x2(v[i][3] * p, v[i][7] * p)};
-            *reinterpret_cast<u32x4_t*>(x16 + static_cast<size_t>(m) * cols + 8 * b) = h;
+        const int b = i0 + 64 * WPT * i;
+        if (TPB == 1 && b >= nb) break;
+        const u32x4_t h{pack_f16x2(v[i][0] * p, v[i][4] * p), pack_f16x2(v[i][1] * p, v[i][5] * p),
+                        pack_f16x2(v[i][2] * p, v[i][6] * p), pack_f16x2(v[i][3] * p, v[i][7] * p)};
+        if constexpr (TPB == 1) {
+            *reinterpret_cast<u32x4_t*>(x16 + q4_x16_at(mt, b, G)) = h;
+        } else {
+            if (64 * i >= nb) break;   // workgroup-uniform
+            xo[i & 1][lane * (TPB + 1) + wave] = h;
+            __syncthreads();
+            const int pc = static_cast<int>(threadIdx.x) / TPB, tk = threadIdx.x % TPB, mo = blockIdx.x * TPB + tk;
+            if (64 * i + pc < nb && mo < batch)
+                *reinterpret_cast<u32x4_t*>(x16 + q4_x16_at(mo, 64 * i + pc, G)) = xo[i & 1][pc * (TPB + 1) + tk];
         }
     }
-    if (NORM) {
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) ss += __shfl_xor(ss, o, 64);
-    }
-    if (lane == 0) {
+    if (i0 == 0 && mt < batch) {
         const float rs = NORM ? rsqrtf(ss / static_cast<float>(cols) + nrm.eps) : 1.0f;
         fm[m] = ldexpf(rs, e - 8);
     }
@@ -1063,17 +1104,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         sbl[g * kQ4GemmRows + r] = pack_f16x2(256.0f * elem<SB_DT>::load(scales, gi), 256.0f * elem<SB_DT>::load(biases, gi));
     }
 
-    // x16 staging straight from global memory into LDS: wave w's load i fills
-    // tokens 8 (4w + i) .. +7 of the [128][64] tile, lane l the 16-byte
-    // piece l & 7 of token l >> 3, which holds the token's 8-column block
-    // (l & 7) ^ ((token >> 1) & 7) of the group (the swizzle spreads the 32
-    // rows of an operand read over the bank groups)
-    const uint16_t* xsrc[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int tok = 8 * (4 * wave + i) + (lane >> 3);
-        xsrc[i] = x16 + static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 8 * ((lane & 7) ^ ((tok >> 1) & 7));
-    }
+    // x16 staging straight from global memory into LDS: wave w copies the four
+    // operand blocks (steps ks) of token tile w of the group, lane order kept
+    const int xtile = min(M0 / 32 + wave, (batch - 1) / 32);
+    const uint16_t* xsrc = x16 + static_cast<size_t>(xtile) * G * 2048 + 8 * lane;
     // weight words: lane -> rows 64 wave + 32 rt + r, words 4h .. 4h + 3 of each group
     // (rows past the part's end read its last row; their outputs are not stored)
     const int r = lane & 31, h = lane >> 5;
@@ -1085,8 +1119,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     auto stage_x = [&](int buf, int g) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc[i] + 64 * g),
-                                             (__attribute__((address_space(3))) void*)&Xl[buf][8 * (4 * wave + i) * 64],
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc + 2048 * g + 512 * i),
+                                             (__attribute__((address_space(3))) void*)&Xl[buf][512 * (4 * wave + i)],
                                              16, 0, 0);
     };
     auto fetch_w = [&](u32x4_t (&dst)[2], int g) {
@@ -1124,11 +1158,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         uint32_t sb[2];
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) sb[rt] = sbl[g * kQ4GemmRows + 64 * wave + 32 * rt + r];
-        // B operand of token tile mt, step ks: token 32 mt + r, x16 piece
-        // 4h + ks (swizzled by (token / 2) % 8, so the 32 rows of a read
-        // meet every bank group twice)
-        const uint16_t* xb = &Xl[g & 1][r * 64];
-        const int sw = (r >> 1) & 7;
+        const uint16_t* xb = &Xl[g & 1][8 * lane];   // B operand of token tile mt, step ks: block 4 mt + ks
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             u32x4_t A[2], B[4];
@@ -1136,7 +1166,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
             for (int rt = 0; rt < 2; ++rt) A[rt] = q4_to_f16_scaled(cur[rt][ks], sb[rt], e1024);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
-                B[mt] = *reinterpret_cast<const u32x4_t*>(xb + 32 * mt * 64 + 8 * ((4 * h + ks) ^ sw));
+                B[mt] = *reinterpret_cast<const u32x4_t*>(xb + 512 * (4 * mt + ks));
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
@@ -1186,6 +1216,201 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
                     }
                 }
             }
+    }
+}
+
+// ---- many-token product of short batches: K split over a workgroup's waves --------
+//
+// Below a few hundred tokens the kernel above has too few 256 x 128 tiles for
+// the chip (8 workgroups for 2048 rows x 128 tokens, each walking all of K
+// behind one barrier per group: 1.4 us a group, 90 us at 4096 columns). What
+// bounds this one at 200 tokens x 2048 x 4096 (11 us beside the x16 pass's 5)
+// is the chain of a workgroup's first loads, its four to eight steps of one L2
+// latency each and the reduction; two steps in flight instead of one, or
+// eight waves a workgroup, were not faster except at one tile a wave. Here
+// a workgroup takes 32 RT rows x 32 MT tokens and its WK waves split K: wave
+// wk walks group pairs wk, wk + WK, .. on its own, no barrier in the loop. The
+// x16 operands come straight from L2 into registers (1 KB contiguous each);
+// a pair's weights (64 bytes per row, read by quads of lanes) are turned into
+// the operand order through the wave's own LDS; the waves' sums meet in LDS
+// in wave order at the end. Same operands and products as above.
+template <int SB_DT, int RT, int MT, int WK, int D>
+__global__ __launch_bounds__(64 * WK) __attribute__((amdgpu_waves_per_eu(2))) void q4_gemm_split_kernel(Q4Parts parts, const uint16_t* __restrict__ x16,
+                                                                const float* __restrict__ fm, int cols, int batch,
+                                                                int pmagic) {
+    constexpr int RW = 32 * RT;
+    const int t = threadIdx.x, lane = t & 63, wk = t >> 6;
+    const int r = lane & 31, h = lane >> 5;
+    const Q4Part1 P = q4_part_of(parts, static_cast<int>(blockIdx.x));
+    const int rows = P.rows, R0 = (static_cast<int>(blockIdx.x) - P.blk0) * RW, M0 = static_cast<int>(blockIdx.y) * 32 * MT;
+    const int G = cols / 64, NP = G / 2;
+
+    // packed fp16 (256 s, 256 b) [G][RW + 1] and the waves' turn buffers; at the
+    // end the waves' sums of one token tile, [WK][4 RT][66] 16-byte slots
+    constexpr int RS = RW + 1, kSb = (64 * RS + 3) / 4 * 4, kTurn = WK * RW * 16, kRed = WK * RT * 4 * 66 * 4;
+    __shared__ __attribute__((aligned(16))) uint32_t lds[kSb + kTurn > kRed ? kSb + kTurn : kRed];
+    uint32_t* const sbl = lds;
+    uint32_t* const turn = lds + kSb + wk * RW * 16;
+
+    const uint32_t* wrow[2 * RT];
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i)
+        wrow[i] = P.w + static_cast<size_t>(min(R0 + 16 * i + (lane >> 2), rows - 1)) * (cols / 8) + 4 * (lane & 3);
+    const uint16_t* xsrc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+        xsrc[i] = x16 + static_cast<size_t>(min(M0 / 32 + i, (batch - 1) / 32)) * G * 2048 + 8 * lane;
+    u32x4_t wr[D][2 * RT], xr[D][2][MT][4];
+    auto fetch_w = [&](int s, int p) {
+#pragma unroll
+        for (int i = 0; i < 2 * RT; ++i) wr[s][i] = *reinterpret_cast<const u32x4_t*>(wrow[i] + 16 * p);
+    };
+    auto fetch_x = [&](int s, int gg, int p) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                xr[s][gg][i][ks] = *reinterpret_cast<const u32x4_t*>(xsrc[i] + 2048 * (2 * p + gg) + 512 * ks);
+    };
+#pragma unroll
+    for (int s = 0; s < D; ++s) {
+        fetch_w(s, min(wk + s * WK, NP - 1));
+        fetch_x(s, 0, min(wk + s * WK, NP - 1));
+        fetch_x(s, 1, min(wk + s * WK, NP - 1));
+    }
+    // scales and biases: two groups of a row per 4-byte load
+    constexpr int SBT = RW * 32 / (64 * WK);
+    uint32_t sreg[SBT], breg[SBT];
+#pragma unroll
+    for (int k = 0; k < SBT; ++k) {
+        const int idx = min(t + 64 * WK * k, RW * NP - 1), rr = (idx * pmagic) >> 20;
+        const size_t o = static_cast<size_t>(min(R0 + rr, rows - 1)) * NP + (idx - rr * NP);
+        sreg[k] = reinterpret_cast<const uint32_t*>(P.s)[o];
+        breg[k] = reinterpret_cast<const uint32_t*>(P.b)[o];
+    }
+    // the residuals and factors of the outputs this thread stores at the end
+    // (four adjacent rows of one token per unit), requested now
+    constexpr int NU = (RT * 256 + 64 * WK - 1) / (64 * WK);   // units per thread and token tile
+    const bool rvec = (rows & 3) == 0 && (reinterpret_cast<uintptr_t>(P.res) & 15) == 0;
+    f32x4_t resv[MT][NU];
+    float fmv[MT][NU];
+#pragma unroll
+    for (int b = 0; b < MT; ++b)
+#pragma unroll
+        for (int k = 0; k < NU; ++k) {
+            const int u = t + 64 * WK * k, m = min(M0 + 32 * b + ((u >> 3) & 31), batch - 1);
+            const int rr = min(R0 + 32 * (u >> 8) + 4 * (u & 7), max(rows - 4, 0));
+            resv[b][k] = q4_res4(P, rvec ? static_cast<size_t>(m) * rows + rr : 0, rvec);
+            fmv[b][k] = fm[m];
+        }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int k = 0; k < SBT; ++k) {
+        const int idx = min(t + 64 * WK * k, RW * NP - 1), rr = (idx * pmagic) >> 20, p = idx - rr * NP;
+        uint16_t s2[2] = {static_cast<uint16_t>(sreg[k]), static_cast<uint16_t>(sreg[k] >> 16)};
+        uint16_t b2[2] = {static_cast<uint16_t>(breg[k]), static_cast<uint16_t>(breg[k] >> 16)};
+        sbl[(2 * p) * RS + rr] = pack_f16x2(256.0f * elem<SB_DT>::load(s2, 0), 256.0f * elem<SB_DT>::load(b2, 0));
+        sbl[(2 * p + 1) * RS + rr] = pack_f16x2(256.0f * elem<SB_DT>::load(s2, 1), 256.0f * elem<SB_DT>::load(b2, 1));
+    }
+    asm volatile("" ::: "memory");
+    __syncthreads();
+
+    f32x16_t acc[RT][MT];
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int b = 0; b < MT; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.0f;
+    uint32_t e1024 = 0x64006400u;
+    asm volatile("" : "+v"(e1024));
+    auto step = [&](int s, int p) {
+        // row 16 i + l / 4, piece l % 4 -> 64 bytes a row, the pieces rotated by
+        // (row / 4) % 4 so 16 lanes meet every bank group both ways
+#pragma unroll
+        for (int i = 0; i < 2 * RT; ++i)
+            *reinterpret_cast<u32x4_t*>(turn + (16 * i + (lane >> 2)) * 16 + 4 * ((lane & 3) ^ (lane >> 4))) = wr[s][i];
+        __builtin_amdgcn_wave_barrier();
+        u32x4_t wq[2][RT];
+#pragma unroll
+        for (int gg = 0; gg < 2; ++gg)
+#pragma unroll
+            for (int a = 0; a < RT; ++a)
+                wq[gg][a] = *reinterpret_cast<const u32x4_t*>(turn + (32 * a + r) * 16 + 4 * ((2 * gg + h) ^ ((r >> 2) & 3)));
+        __builtin_amdgcn_wave_barrier();
+        const int pn = min(p + D * WK, NP - 1);   // (the last pair again at the end: no branch around loads)
+        fetch_w(s, pn);
+#pragma unroll
+        for (int gg = 0; gg < 2; ++gg) {
+            uint32_t sb[RT];
+#pragma unroll
+            for (int a = 0; a < RT; ++a) sb[a] = sbl[(2 * p + gg) * RS + 32 * a + r];
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                u32x4_t A[RT];
+#pragma unroll
+                for (int a = 0; a < RT; ++a) A[a] = q4_to_f16_scaled(wq[gg][a][ks], sb[a], e1024);
+#pragma unroll
+                for (int a = 0; a < RT; ++a)
+#pragma unroll
+                    for (int b = 0; b < MT; ++b) acc[a][b] = mfma_32x32x16_f16(A[a], xr[s][gg][b][ks], acc[a][b]);
+            }
+            fetch_x(s, gg, pn);
+        }
+        asm volatile("" ::: "memory");   // the requests stay in this step
+    };
+    for (int p = wk; p < NP; p += D * WK) {   // wave-uniform
+        step(0, p);
+        if (D > 1 && p + WK < NP) step(D - 1, p + WK);
+    }
+
+    // per token tile: the waves' sums through LDS (slot 33 h + r of each
+    // register quad), added in wave order; eight lanes then hold 32 adjacent
+    // rows of one token
+    f32x4_t* const red = reinterpret_cast<f32x4_t*>(lds);
+    const bool has_res = P.res != nullptr, ybf = P.ybf16 != 0;
+#pragma unroll
+    for (int b = 0; b < MT; ++b) {
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < RT; ++a)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                red[((wk * RT + a) * 4 + j) * 66 + 33 * h + r] =
+                    f32x4_t{acc[a][b][4 * j], acc[a][b][4 * j + 1], acc[a][b][4 * j + 2], acc[a][b][4 * j + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NU; ++k) {
+            const int u = t + 64 * WK * k;
+            if (u >= RT * 256) break;
+            const int q = u & 7, tk = (u >> 3) & 31, a = u >> 8;
+            const int m = M0 + 32 * b + tk, rr = R0 + 32 * a + 4 * q;
+            f32x4_t v = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int w = 0; w < WK; ++w) v += red[((w * RT + a) * 4 + (q >> 1)) * 66 + 33 * (q & 1) + tk];
+            if (m >= batch) continue;
+            const size_t o = static_cast<size_t>(m) * rows + rr;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] *= fmv[b][k];
+                if (rvec) v[i] += resv[b][k][i];   // zero without a residual
+                else if (has_res && rr + i < rows) v[i] += ybf ? elem<1>::load(P.res, o + i) : elem<0>::load(P.res, o + i);
+            }
+            if (rr + 3 < rows && (rows & 3) == 0) {
+                if (ybf)
+                    *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(P.y) + o) =
+                        u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+                else
+                    *reinterpret_cast<f32x4_t*>(static_cast<float*>(P.y) + o) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (rr + i >= rows) continue;
+                    if (ybf) elem<1>::store(P.y, o + i, v[i]);
+                    else elem<0>::store(P.y, o + i, v[i]);
+                }
+            }
+        }
     }
 }
 
@@ -1256,10 +1481,14 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
         const void* xm = static_cast<const char*>(x) + static_cast<size_t>(m0) * cols * (x_dtype == QFF_BF16 ? 2 : 4);
         {
             ProfScope prof(ctx, stream, "q4_x16");
-            if (x_dtype == QFF_BF16)
-                q4_x16_kernel<1, NORM><<<(mb + 3) / 4, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);
-            else
-                q4_x16_kernel<0, NORM><<<(mb + 3) / 4, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);
+            // four waves a token below 768 tokens (2048 x 4096 product, both
+            // launches: 11.3 against 12.3 us at 33, 16.4 / 17.3 at 200; equal at
+            // 768, 140 / 131 at 4096)
+#define QFF_X16(X)                                                                                                       \
+    if (mb < 768) q4_x16_kernel<X, NORM, 4, 1><<<mb, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);     \
+    else q4_x16_kernel<X, NORM, 1, 8><<<(mb + 7) / 8, 512, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm)
+            if (x_dtype == QFF_BF16) { QFF_X16(1); } else { QFF_X16(0); }
+#undef QFF_X16
         }
         // one launch over every part's row tiles, outputs offset to this slice
         qff_q4_part sl[QFF_Q4_MAX_PARTS];
@@ -1269,14 +1498,55 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
             sl[i].y = static_cast<char*>(parts[i].y) + yoff;
             if (parts[i].residual) sl[i].residual = static_cast<const char*>(parts[i].residual) + yoff;
         }
-        int tiles = 0;
-        const Q4Parts P = q4_pack_parts(sl, nparts, kQ4GemmRows, tiles);
-        const dim3 grid(tiles, (mb + kQ4GemmToks - 1) / kQ4GemmToks);
+        const auto pack_grid = [&](int rpb, int tpb, Q4Parts& P) {
+            int tiles = 0;
+            P = q4_pack_parts(sl, nparts, rpb, tiles);
+            return dim3(tiles, (mb + tpb - 1) / tpb);
+        };
+        const auto count = [](dim3 g) { return static_cast<int>(g.x * g.y); };
+        // Which kernel: by the tokens and columns alone, and K always split in
+        // four, so that a part's sums do not depend on the rows beside it
+        // (scales and biases are read two groups at a time: an even number of
+        // groups, 4-byte-aligned scale rows). Which tile: the largest that
+        // still covers the chip. fp32 x, x16 pass included, us at 64 / 200 /
+        // 512 / 1000 / 4096 tokens:
+        //   2048 x 4096, 256 x 128 tiles    73 / 97 / 99 / 99 / 152
+        //     K split 32 x 32               12 / 18 / 29 / 51
+        //     K split 32 x 64               13 / 17 / 25 / 43 / 154
+        //     K split 64 x 64               17 / 21 / 25 / 37 / 128
+        //   12352 x 2048, 256 x 128 tiles   45 / 50 / 53 / 79 / 260
+        //     K split 32 x 64               15 / 34 / 61
+        //     K split 64 x 64               15 / 33 / 57 / 100
+        // The large tile stages the scales of all of K in LDS and so runs one
+        // workgroup a CU above 2048 columns: it takes over later there.
+        Q4Parts P;
         ProfScope prof(ctx, stream, "q4_gemm");
-        if (sb_dtype == QFF_BF16)
-            q4_gemm_kernel<1><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
-        else
-            q4_gemm_kernel<2><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
+        const int cu = ctx->num_cu, pm = (1 << 20) / std::max(G / 2, 1) + 1;   // idx / (G / 2) = idx pm >> 20, idx < 2048
+        bool split = G % 2 == 0;
+        for (int i = 0; i < nparts; ++i)
+            split = split && ((reinterpret_cast<uintptr_t>(sl[i].scales) | reinterpret_cast<uintptr_t>(sl[i].biases)) & 3) == 0;
+        split = split && batch <= (cols > 2048 ? 4096 : 512);
+        dim3 grid;
+#define QFF_SPLIT(RT, MT, WK, D)                                                                               \
+    if (sb_dtype == QFF_BF16)                                                                                  \
+        q4_gemm_split_kernel<1, RT, MT, WK, D><<<grid, 64 * WK, 0, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb, pm); \
+    else                                                                                                       \
+        q4_gemm_split_kernel<2, RT, MT, WK, D><<<grid, 64 * WK, 0, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb, pm)
+        if (!split) {
+            grid = pack_grid(kQ4GemmRows, kQ4GemmToks, P);
+            if (sb_dtype == QFF_BF16)
+                q4_gemm_kernel<1><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
+            else
+                q4_gemm_kernel<2><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
+        } else if (count(grid = pack_grid(32, 32, P)) <= cu) {
+            QFF_SPLIT(1, 1, 4, 2);
+        } else if (count(grid = pack_grid(32, 64, P)) <= cu) {
+            QFF_SPLIT(1, 2, 4, 1);
+        } else {
+            grid = pack_grid(64, 64, P);
+            QFF_SPLIT(2, 2, 4, 1);
+        }
+#undef QFF_SPLIT
     }
     return hipGetLastError();
 }

@@ -324,6 +324,45 @@ def test_q4_matmul_parts_4096_cols_f32_x_residual(hip, batch):
             assert _rel(to_np(outs[i]), ref) <= (1e-5 if dt == torch.float32 else 4e-3)
 
 
+@pytest.mark.parametrize("batch,cols,odd", [
+    (33, 128, False), (64, 4096, False), (65, 2048, False),     # one pair of groups; whole and ragged token tiles
+    (200, 1152, False), (512, 2048, False), (513, 2048, False),  # the last batch of the split kernel and the next
+    (70, 2048, True), (40, 192, False),                          # odd scale addresses; an odd number of groups
+    (800, 4096, False),                                          # eight tokens a workgroup in the fp16 pass
+])
+def test_q4_many_tokens_split_tiles(hip, batch, cols, odd):
+    """The many-token product at the edges of its tiles: three parts (whole
+    tiles, a ragged one, one of 3 rows), fp32 and bf16 outputs, a residual in
+    place, the input norm; within 1e-3 (fp16 operands, 2^-12 each: 3e-4
+    expected) of the fp64 product, bf16 outputs 4e-3."""
+    import qff
+    print(f"q4 many tokens batch={batch} cols={cols} odd={odd}", flush=True)
+    shapes = [(256, torch.float32), (100, torch.bfloat16), (3, torch.float32)]
+    ws = [synth.q4_weight(r, cols, seed=r + batch) for r, _ in shapes]
+    rng = np.random.default_rng(batch + cols)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    nw = (1 + 0.1 * rng.standard_normal(cols)).astype(np.float32)
+    res = [(30 * rng.standard_normal((batch, r))).astype(np.float32) for r, _ in shapes]
+
+    def gpu(w, s, b):
+        w, s, b = _w_gpu(w, s, b, "f16")
+        if odd:   # scale rows at 2 bytes past a 4-byte boundary
+            s, b = (torch.cat([v.new_zeros(1), v.flatten()])[1:].view(v.shape) for v in (s, b))
+        return w, s, b
+
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=64)
+    ys = [f32_tensor(res[0]), torch.empty(batch, 100, dtype=torch.bfloat16, device=DEV), f32_tensor(res[2])]
+    outs = qff.q4_norm_matmul_parts(ctx, [gpu(*w) for w in ws], f32_tensor(x), f32_tensor(nw), 1e-6, outs=ys,
+                                    residuals=[ys[0], None, ys[2]])
+    torch.cuda.synchronize()
+    x64 = x.astype(np.float64)
+    xn = x64 / np.sqrt(np.mean(x64 ** 2, axis=1, keepdims=True) + 1e-6) * nw
+    for i, (w, (_, dt)) in enumerate(zip(ws, shapes)):
+        ref = xn @ O.q4_dequant(*w, O.F16).astype(np.float64).T
+        got = to_np(outs[i]).astype(np.float64) - (0 if i == 1 else res[i])
+        assert _rel(got, ref) <= (1e-3 if dt == torch.float32 else 4e-3)
+
+
 def test_q4_norm_matmul_parts_rejects_bad_calls(hip):
     import qff
     from qff._lib import Q4Part, lib
