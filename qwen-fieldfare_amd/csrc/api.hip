@@ -26,6 +26,12 @@ static qff_ctx_cfg resolve(const qff_ctx_cfg* cfg) {
 // Tokens per slice of a many-token Q4 product (fp16 activations in workspace).
 int q4_xs_tokens(const qff_ctx_cfg& cfg) { return std::max(std::max(cfg.max_batch, cfg.max_prefill_tokens), 1024); }
 
+int pf_slots(const qff_ctx_cfg& cfg) {
+    const long long tc = (static_cast<long long>(cfg.max_prefill_tokens) + 63) / 64 * 64;
+    const long long tiles = (static_cast<long long>(cfg.max_ctx) + 63) / 64;
+    return static_cast<int>(std::max(tc, std::min(3072ll, tc * std::max(1ll, tiles / 4))));
+}
+
 WorkspaceLayout workspace_layout(const qff_ctx_cfg& cfg) {
     WorkspaceLayout L{};
     size_t off = 0;
@@ -43,7 +49,9 @@ WorkspaceLayout workspace_layout(const qff_ctx_cfg& cfg) {
     L.q4_fm = take(static_cast<size_t>(q4_xs_tokens(cfg)) * sizeof(float));
     L.q4_sk_part = take(static_cast<size_t>(kQ4SkSlots) * 16 * 64 * sizeof(float));
     const size_t TC = (T + 63) / 64 * 64;   // tokens rounded up to whole chunks
-    L.pf_o = take(TC * 4096 * sizeof(float));   // pre-norm DeltaNet prefill output, fp32
+    const size_t PS = static_cast<size_t>(pf_slots(cfg));   // >= TC
+    L.pf_o = take(PS * 4096 * sizeof(float));   // pre-norm DeltaNet prefill output, or prefill attention partials, fp32
+    L.pf_md = take(PS * 32 * sizeof(float));
     L.sched = take(2 * kSchedSlots * sizeof(unsigned));
     L.dn_arrive = take(B * 16 * sizeof(unsigned));
     // DeltaNet prefill chunk records (deltanet_chunked.hip): per chunk and key
@@ -170,6 +178,8 @@ int qff_ctx_create(qff_ctx** out, int device, const qff_ctx_cfg* cfg) {
     c->q4_xs_tokens = q4_xs_tokens(c->cfg);
     c->q4_sk_part = reinterpret_cast<float*>(base + L.q4_sk_part);
     c->pf_o = reinterpret_cast<float*>(base + L.pf_o);
+    c->pf_md = reinterpret_cast<float*>(base + L.pf_md);
+    c->pf_slots = pf_slots(c->cfg);
     c->sched = reinterpret_cast<unsigned*>(base + L.sched);
     c->num_cu = prop.multiProcessorCount;
     c->dn_arrive = reinterpret_cast<unsigned*>(base + L.dn_arrive);

@@ -36,6 +36,8 @@
 //          are issued last-first so the longest rows start earliest. The
 //          epilogue merges each pair's halves, divides by the row sums and
 //          applies the sigmoid gate.
+#include <algorithm>
+
 #include "common.hpp"
 #include "internal.hpp"
 #include "mfma.hpp"
@@ -325,10 +327,17 @@ __device__ __forceinline__ void phase_barrier() {
 // V_{kt-2} left), straight into LDS, waiting for them before the next
 // barrier. All eight waves run the same schedule, two per SIMD, so one
 // wave's operand reads and softmax overlap the other's MFMAs.
-template <int IN_DT, int OUT_DT>
+//
+// SPLIT: blockIdx.z walks its share of the block's tiles only and stores the
+// rows' running maximum, sum and unnormalised O^T (fp32) for
+// gqa_prefill_combine_kernel: blocks of few tokens behind a long cache, which
+// alone would leave most CUs idle (500 tokens behind 12011: 64 workgroups of
+// 196 tiles, 268 us; in four shares 256 of 49).
+template <int IN_DT, int OUT_DT, bool SPLIT>
 __global__ __launch_bounds__(kPfThreads) void gqa_prefill_attn_kernel(
     const uint16_t* __restrict__ qb, const void* __restrict__ q_gate, const uint16_t* __restrict__ k16,
-    const uint16_t* __restrict__ vt, int vt_stride, int start, int T, void* __restrict__ out) {
+    const uint16_t* __restrict__ vt, int vt_stride, int start, int T, void* __restrict__ out,
+    float2* __restrict__ part_md, float* __restrict__ part_o) {
     // K tiles 0, 1 and V^T tiles 0, 1 (kvs[2], kvs[3]); after the loop,
     // each wave's 16 KB hand-over of O^T to its partner
     __shared__ __attribute__((aligned(1024))) uint16_t kvs[4][kPfKT * 256];
@@ -343,6 +352,23 @@ __global__ __launch_bounds__(kPfThreads) void gqa_prefill_attn_kernel(
     const int pr = wave >> 1, e = wave & 1, partner = wave ^ 1;
     constexpr float kLazy = 8.0f;   // raise the running max only past 2^8
 
+    int kv_end = start + min(T, t0 + kPfQB);
+    int ntiles = (kv_end + kPfKT - 1) / kPfKT;
+    if constexpr (SPLIT) {
+        // this workgroup's tiles base .. base + ntiles - 1 (every share has
+        // one: the launch has no more shares than its first block tiles);
+        // from here on positions count from the first of them
+        const int z = static_cast<int>(blockIdx.z), nz = static_cast<int>(gridDim.z);
+        const int base = ntiles * z / nz;
+        ntiles = ntiles * (z + 1) / nz - base;
+        start -= base * kPfKT;
+        kv_end -= base * kPfKT;
+        k16 += static_cast<size_t>(base) * (kPfKT * 512);
+        vt += static_cast<size_t>(base) * (kPfKT * 256);
+    }
+    // tiles before this need no causal mask (below zero: all of a share do)
+    const int first_masked = start + t0 >= 0 ? (start + t0) / kPfKT : 0;
+
     // the lane's q row: token t0 + 4 pr + r / 8, head r % 8; B operand of S
     // step s = dims 16s + 8h .. +7
     const int tok_q = min(t0 + 4 * pr + (r >> 3), T - 1);
@@ -356,10 +382,6 @@ __global__ __launch_bounds__(kPfThreads) void gqa_prefill_attn_kernel(
 #pragma unroll
         for (int s = 0; s < 16; ++s) asm volatile("" ::"v"(qreg[s]));
     }
-    const int kv_end = start + min(T, t0 + kPfQB);
-    const int ntiles = (kv_end + kPfKT - 1) / kPfKT;
-    const int first_masked = (start + t0) / kPfKT;   // tiles before this need no causal mask
-
     float m_run = -INFINITY, d_run = 0.0f;   // of the lane's row (the same in lanes r, r + 32)
     f32x16_t oacc[8];                        // O^T tile dt: dims 32dt + 8(i/4) + 4h + i%4
 #pragma unroll
@@ -555,8 +577,10 @@ __global__ __launch_bounds__(kPfThreads) void gqa_prefill_attn_kernel(
         __syncthreads();
         const float mp = xm[partner][r], dp = xd[partner][r];
         const float mx = fmaxf(m_run, mp);
-        const float fo = __builtin_amdgcn_exp2f(m_run - mx), fp = __builtin_amdgcn_exp2f(mp - mx);
-        const float inv_d = 1.0f / (d * fo + dp * fp);
+        // (a share may hold no position of a row: maximum -inf, sum zero)
+        const float mf = SPLIT && mx == -INFINITY ? 0.0f : mx;
+        const float fo = __builtin_amdgcn_exp2f(m_run - mf), fp = __builtin_amdgcn_exp2f(mp - mf);
+        const float inv_d = SPLIT ? 1.0f : 1.0f / (d * fo + dp * fp);
         const float so = fo * inv_d, sp = fp * inv_d;
         const f32x4_t* const xq = reinterpret_cast<const f32x4_t*>(kvs[0]) + partner * 1024;
         const int tok = t0 + 4 * pr + (r >> 3);
@@ -564,12 +588,21 @@ __global__ __launch_bounds__(kPfThreads) void gqa_prefill_attn_kernel(
             constexpr int E = decltype(ev)::value;
             if (tok >= T) return;
             const size_t qi = static_cast<size_t>(tok) * 16 + kvh * 8 + (r & 7);
+            const size_t pi = SPLIT ? static_cast<size_t>(blockIdx.z) * T * 16 + qi : 0;   // partial row
+            if (SPLIT && E == 0 && h == 0) part_md[pi] = make_float2(mx, d * fo + dp * fp);
 #pragma unroll
             for (int c = 0; c < 4; ++c)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int dim = 128 * E + 32 * c + 8 * j + 4 * h;
                     const f32x4_t po = xq[(4 * c + j) * 64 + lane];
+                    if constexpr (SPLIT) {
+                        f32x4_t v;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) v[i] = oacc[4 * E + c][4 * j + i] * so + po[i] * sp;
+                        *reinterpret_cast<f32x4_t*>(part_o + pi * 256 + dim) = v;
+                        continue;
+                    }
                     float g[4], y[4];
                     if constexpr (IN_DT == 1) {
                         const u32x2_t w = *reinterpret_cast<const u32x2_t*>(
@@ -599,6 +632,51 @@ __global__ __launch_bounds__(kPfThreads) void gqa_prefill_attn_kernel(
         if (e == 0) finish(std::integral_constant<int, 0>{});
         else finish(std::integral_constant<int, 1>{});
     }
+}
+
+// One wave per (token, q head): the shares' rows weighted by exp2(m_s - max m),
+// over the weighted sum, * sigmoid(gate); lane l holds dims 4l .. 4l + 3.
+template <int IN_DT, int OUT_DT>
+__global__ __launch_bounds__(256) void gqa_prefill_combine_kernel(const float2* __restrict__ part_md,
+                                                                  const float* __restrict__ part_o,
+                                                                  const void* __restrict__ q_gate, int T, int shares,
+                                                                  void* __restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    const size_t row = static_cast<size_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), rows = static_cast<size_t>(T) * 16;
+    if (row >= rows) return;   // wave-uniform
+    float g[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) g[i] = elem<IN_DT>::load(q_gate, row * 512 + 256 + 4 * lane + i);
+    // share lane's (m, d); shares <= 64
+    const float2 md = part_md[static_cast<size_t>(min(lane, shares - 1)) * rows + row];
+    const bool mine = lane < shares;
+    const float mx = group_max<64>(mine ? md.x : -INFINITY);
+    const float w = mine && md.y > 0.0f ? __builtin_amdgcn_exp2f(md.x - mx) : 0.0f;
+    const float inv_d = 1.0f / group_sum<64>(w * md.y);
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    constexpr int U = 4;   // rows requested together
+    for (int s0 = 0; s0 < shares; s0 += U) {
+        f32x4_t o[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            o[u] = *reinterpret_cast<const f32x4_t*>(
+                part_o + (static_cast<size_t>(min(s0 + u, shares - 1)) * rows + row) * 256 + 4 * lane);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const float ws = s0 + u < shares ? __shfl(w, s0 + u, 64) : 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i] = fmaf(ws, o[u][i], acc[i]);
+        }
+    }
+    const size_t oi = row * 256 + 4 * lane;
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = acc[i] * inv_d * sigmoid(g[i]);
+    if constexpr (OUT_DT == 1)
+        *reinterpret_cast<u32x2_t*>(static_cast<uint16_t*>(out) + oi) =
+            u32x2_t{pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])};
+    else
+        *reinterpret_cast<f32x4_t*>(static_cast<float*>(out) + oi) = f32x4_t{y[0], y[1], y[2], y[3]};
 }
 
 hipError_t launch_gqa_prefill(qff_ctx* ctx, hipStream_t stream, const qff_gqa_params* p,
@@ -639,17 +717,44 @@ hipError_t launch_gqa_prefill(qff_ctx* ctx, hipStream_t stream, const qff_gqa_pa
 #undef QFF_PREP
     }
     const int vt_stride = (ctx->cfg.max_ctx + kPfKT - 1) / kPfKT;
-    const dim3 grid((T + kPfQB - 1) / kPfQB, 2);
-    ProfScope prof(ctx, stream, "gqa_prefill_attn");
-#define QFF_PFA(I, O) \
-    gqa_prefill_attn_kernel<I, O><<<grid, kPfThreads, 0, stream>>>(qb, q_gate, k16, ctx->gqa_vt, vt_stride, \
-                                                                   start_pos, T, out)
-    if (in_dtype == QFF_BF16) {
-        if (out_dtype == QFF_BF16) QFF_PFA(1, 1); else QFF_PFA(1, 0);
-    } else {
-        if (out_dtype == QFF_BF16) QFF_PFA(0, 1); else QFF_PFA(0, 0);
-    }
+    const int nqb = (T + kPfQB - 1) / kPfQB, ntiles = (start_pos + T + kPfKT - 1) / kPfKT;
+    // Shares of the tiles per block: enough to give every CU one workgroup, of
+    // four tiles or more each, no more than the first block has tiles (none is
+    // empty; a prompt from position 0 is not shared) nor than the partial
+    // slots. us per call, one share / this rule / the best of 1 .. 64:
+    //   16 tokens at 2000, 12000, 60000   64 / 31 / 30, 253 / 39 / 39, 1477 / 82 / 82
+    //   128 at 2000, 12000                69 / 37 / 37, 257 / 61 / 60
+    //   500 at 3000, 12011                97 / 59 / 59, 265 / 129 / 129
+    //   1000 at 2000, 8000                88 / 76 / 76, 201 / 168 / 168
+    int shares = std::min(std::min(ctx->num_cu / (2 * nqb), ntiles / 4), std::min(64, start_pos / kPfKT + 1));
+    shares = std::max(1, std::min(shares, ctx->pf_slots / T));
+    float2* md = reinterpret_cast<float2*>(ctx->pf_md);
+    {
+        ProfScope prof(ctx, stream, "gqa_prefill_attn");
+        const dim3 grid(nqb, 2, shares);
+#define QFF_PFA(I, O, SP) \
+    gqa_prefill_attn_kernel<I, O, SP><<<grid, kPfThreads, 0, stream>>>(qb, q_gate, k16, ctx->gqa_vt, vt_stride, start_pos, \
+                                                                       T, out, md, ctx->pf_o)
+        if (shares > 1) {
+            QFF_PFA(1, 1, true);   // (reads no gate and writes no output)
+        } else if (in_dtype == QFF_BF16) {
+            if (out_dtype == QFF_BF16) QFF_PFA(1, 1, false); else QFF_PFA(1, 0, false);
+        } else {
+            if (out_dtype == QFF_BF16) QFF_PFA(0, 1, false); else QFF_PFA(0, 0, false);
+        }
 #undef QFF_PFA
+    }
+    if (shares > 1) {
+        ProfScope prof(ctx, stream, "gqa_prefill_combine");
+        const int blocks = T * 4;   // four (token, head) rows each
+#define QFF_PFC(I, O) gqa_prefill_combine_kernel<I, O><<<blocks, 256, 0, stream>>>(md, ctx->pf_o, q_gate, T, shares, out)
+        if (in_dtype == QFF_BF16) {
+            if (out_dtype == QFF_BF16) QFF_PFC(1, 1); else QFF_PFC(1, 0);
+        } else {
+            if (out_dtype == QFF_BF16) QFF_PFC(0, 1); else QFF_PFC(0, 0);
+        }
+#undef QFF_PFC
+    }
     return hipGetLastError();
 }
 

@@ -49,8 +49,12 @@ struct qff_ctx {
     // slice) the partial [16 tokens][64 rows], kQ4SkSlots of them.
     float* q4_sk_part = nullptr;
     // DeltaNet prefill: pre-norm outputs [T rounded up to 64][32][128] fp32
-    // and chunk intermediates.
+    // and chunk intermediates. Full-attention prefill in shares: the partial
+    // O rows [pf_slots][16][256] fp32 of (share, token) slots in the same
+    // bytes, and their (m, d) pairs.
     float* pf_o = nullptr;
+    float* pf_md = nullptr;   // [pf_slots][16][2]
+    int pf_slots = 0;
     qff_dn_bufs dn{};
     // DeltaNet decode: per (sequence, key head) arrival counters [max_batch][16],
     // zero between launches (the second arrival resets its counter).
@@ -72,13 +76,17 @@ constexpr int kGqaSeqChunks = 128;     // partial slots per (sequence, kv head) 
 // (sequence, kv head, chunk) partial slots of the workspace: a call with a
 // smaller batch spreads them over more chunks per sequence.
 inline int gqa_slots(const qff_ctx_cfg& cfg) { return 2 * (cfg.max_batch > 4 ? cfg.max_batch : 4) * kGqaSeqChunks; }
+// (share, token) slots of a full-attention prefill in shares: as many as its
+// longest call can use, 3072 (a share of every CU and half as many again) at
+// most where that exceeds a call's tokens.
+int pf_slots(const qff_ctx_cfg& cfg);
 constexpr int kSchedSlots = 8;         // work-queue counter pairs in the context
 constexpr int kQ4SkSlots = 4096;       // (row tile, slice) partials of the split decode-batch Q4 product
 constexpr int kSchedChunkLocal = 0;    // slot of the DeltaNet chunk-local pass
 
 struct WorkspaceLayout {
     size_t gqa_m, gqa_d, gqa_o;
-    size_t gqa_qb, gqa_kv16, gqa_vt, q4_x16, q4_fm, q4_sk_part, pf_o, dn_arrive, sched, kimg, qop, top, pop, gates, bv;
+    size_t gqa_qb, gqa_kv16, gqa_vt, q4_x16, q4_fm, q4_sk_part, pf_o, pf_md, dn_arrive, sched, kimg, qop, top, pop, gates, bv;
     size_t total;
 };
 WorkspaceLayout workspace_layout(const qff_ctx_cfg& cfg);

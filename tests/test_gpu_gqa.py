@@ -223,6 +223,15 @@ def test_gqa_prefill_matches_token_by_token(hip, T, start):
     _prefill_case(hip, T, start, max_ctx=2048, out_dtype=torch.float32 if T == 17 else torch.bfloat16)
 
 
+@pytest.mark.parametrize("T,start,max_ctx", [(5, 17000, 17024), (33, 511, 576), (250, 256, 512), (40, 1003, 1050)])
+def test_gqa_prefill_in_shares(hip, T, start, max_ctx):
+    """Few tokens behind a cache, the tiles shared out over several workgroups
+    per block: the 64 shares of the longest case, two shares whose boundary
+    and last tile are ragged, a share that lies wholly past a block's first
+    tokens; fp32 outputs within 2e-2 of the oracle, every row."""
+    _prefill_case(hip, T, start, max_ctx, out_dtype=torch.float32, rows=range(0, T, 7) if T > 100 else None, seed=T)
+
+
 def test_gqa_prefill_config3_full_length_sampled_rows(hip):
     """T = 8192 from position 0: every appended K/V entry, and a sample of
     output rows (first, last, tile and block boundaries, random)."""
