@@ -114,3 +114,23 @@ def test_parameter_structs_match_the_header(tmp_path):
         assert int(got[f"{cname} size"]) == ctypes.sizeof(py), cname
         for fname, _ in py._fields_:
             assert int(got[f"{cname} {fname}"]) == getattr(py, fname).offset, (cname, fname)
+
+
+def test_packed_parameter_blocks_match_the_structures():
+    """The bytes ops.py hands over are the ctypes structures', field for field,
+    values past fp32 and non-numbers included."""
+    import ctypes
+    from qff import ops
+    from qff._lib import DeltaNetParams, GqaParams, Q4Part
+    ptrs = [0x1122334455667788 + i for i in range(6)]
+    for eps in (1e-6, 0.0, 1e39, float("inf")):
+        assert ops._pack(ops._P_DN, ptrs[:4], eps) == bytes(DeltaNetParams(*ptrs[:4], eps))
+        assert ops._pack(ops._P_GQA, ptrs[:2], 1e7, 64, 1 / 16, eps, 1) == \
+            bytes(GqaParams(*ptrs[:2], 1e7, 64, 1 / 16, eps, 1))
+    with pytest.raises(TypeError):
+        ops._pack(ops._P_DN, ptrs[:4], "1e-6")
+    parts = [(*ptrs[:3], 100 + i, ptrs[3], i % 2, (None, ptrs[4])[i % 2]) for i in range(8)]
+    for n in range(1, 9):
+        arr = (Q4Part * n)(*(Q4Part(*q) for q in parts[:n]))
+        flat = [0 if v is None else v for q in parts[:n] for v in q]
+        assert ops._P_Q4[n].pack(*flat) == ctypes.string_at(arr, ctypes.sizeof(arr))
