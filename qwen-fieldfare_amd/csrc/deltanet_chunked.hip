@@ -97,16 +97,16 @@ __device__ __forceinline__ int kimg_off(int r, int q) { return r * 128 + ((q ^ (
 template <int IN_DT> struct RawPair;
 template <> struct RawPair<1> {
     uint32_t v;
-    __device__ __forceinline__ void load(const void* p, size_t i) {
-        v = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p) + i);
+    __device__ __forceinline__ void load(const void* p, size_t row, uint32_t i) {
+        v = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p) + row + i);
     }
     __device__ __forceinline__ float lo() const { return __uint_as_float(v << 16); }
     __device__ __forceinline__ float hi() const { return __uint_as_float(v & 0xffff0000u); }
 };
 template <> struct RawPair<0> {
     float2 v;
-    __device__ __forceinline__ void load(const void* p, size_t i) {
-        v = *reinterpret_cast<const float2*>(static_cast<const float*>(p) + i);
+    __device__ __forceinline__ void load(const void* p, size_t row, uint32_t i) {
+        v = *reinterpret_cast<const float2*>(static_cast<const float*>(p) + row + i);
     }
     __device__ __forceinline__ float lo() const { return v.x; }
     __device__ __forceinline__ float hi() const { return v.y; }
@@ -138,19 +138,20 @@ __device__ __forceinline__ void fetch_unit(UnitIn<IN_DT>& in, int u, int T, cons
                                            const float* __restrict__ a, const float* __restrict__ b,
                                            const float* __restrict__ a_log, const float* __restrict__ dt_bias,
                                            const float* __restrict__ conv_w, int wave, int lane) {
+    // unit and wave are uniform, and told so: the 44 row addresses are then
+    // scalar bases with one lane offset per pass instead of vector arithmetic
     int c, kh;
-    unit_coords(u, c, kh);
-    const int t0 = c * kC, tw = t0 + 8 * wave;
-    const int chs[4] = {kh * 128 + 2 * lane, 2048 + kh * 128 + 2 * lane, 4096 + 2 * kh * 128 + 2 * lane,
-                        4096 + (2 * kh + 1) * 128 + 2 * lane};
+    unit_coords(__builtin_amdgcn_readfirstlane(u), c, kh);
+    const int t0 = c * kC, tw = t0 + 8 * __builtin_amdgcn_readfirstlane(wave);
+    const int chb[4] = {kh * 128, 2048 + kh * 128, 4096 + 2 * kh * 128, 4096 + (2 * kh + 1) * 128};
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) in.w[p][j] = reinterpret_cast<const float4*>(conv_w)[chs[p] + j];
+        for (int j = 0; j < 2; ++j) in.w[p][j] = reinterpret_cast<const float4*>(conv_w)[chb[p] + 2 * lane + j];
 #pragma unroll
         for (int i = 0; i < 11; ++i) {
             const int pos = min(max(tw - 3 + i, 0), T - 1);
-            in.r[p][i].load(qkv, static_cast<size_t>(pos) * 8192 + chs[p]);
+            in.r[p][i].load(qkv, static_cast<size_t>(pos) * 8192 + chb[p], 2u * lane);
         }
     }
 #pragma unroll
@@ -204,29 +205,57 @@ __device__ __forceinline__ void conv2x8(const float (&e)[11][2], const float4 (&
 }
 
 // Totals over the 64 lanes of a wave of eight per-lane partials, in every
-// lane: a reduce-scatter (exchanges with lane ^ 32, ^ 16, ^ 8 halve the set
-// each time), the last three butterfly steps, then one readlane per value.
+// lane: a reduce-scatter (the half swap and the row swap leave each lane the
+// two operands of its sum, a row rotation pairs lane ^ 8), the sum of eight
+// lanes, then one readlane per value. Register moves throughout: the same
+// exchanges as LDS permutes took ~130 cycles each, in a chain of six.
 __device__ __forceinline__ void wave_sum8(const float (&p)[8], float (&tot)[8], int lane) {
-    const bool b5 = lane & 32, b4 = lane & 16, b3 = lane & 8;
     float q4[4], q2[2];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float keep = b5 ? p[4 + j] : p[j], give = b5 ? p[j] : p[4 + j];
-        q4[j] = keep + __shfl_xor(give, 32, 64);
+        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[j]), __float_as_uint(p[4 + j]), false, false);
+        q4[j] = __uint_as_float(h[0]) + __uint_as_float(h[1]);   // lanes 0-31 value j, 32-63 value 4 + j
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-        const float keep = b4 ? q4[2 + j] : q4[j], give = b4 ? q4[j] : q4[2 + j];
-        q2[j] = keep + __shfl_xor(give, 16, 64);
+        const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(q4[j]), __float_as_uint(q4[2 + j]), false, false);
+        q2[j] = __uint_as_float(h[0]) + __uint_as_float(h[1]);   // odd rows of 16 value 2 + j on top
     }
-    float q1 = (b3 ? q2[1] : q2[0]) + __shfl_xor(b3 ? q2[0] : q2[1], 8, 64);
-    q1 += __shfl_xor(q1, 4, 64);
-    q1 += __shfl_xor(q1, 2, 64);
-    q1 += __shfl_xor(q1, 1, 64);
+    const bool b3 = lane & 8;
+    float q1 = (b3 ? q2[1] : q2[0]) + dpp_mov<0x128>(b3 ? q2[0] : q2[1]);   // row_ror:8
+    q1 = group_sum<8>(q1);
     // lane L now holds the total of value (L >> 3) & 7
 #pragma unroll
     for (int j = 0; j < 8; ++j)
         tot[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q1), 8 * j));
+}
+
+// Inclusive prefix sum over the wave's lanes: within each row of 16 by row
+// shifts, then the rows' totals (row_bcast:15, row_bcast:31).
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_rows(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xf, true));
+}
+__device__ __forceinline__ float wave_inclusive_scan(float v) {
+    v += dpp_rows<0x111, 0xf>(v);
+    v += dpp_rows<0x112, 0xf>(v);
+    v += dpp_rows<0x114, 0xf>(v);
+    v += dpp_rows<0x118, 0xf>(v);
+    v += dpp_rows<0x142, 0xa>(v);
+    v += dpp_rows<0x143, 0xc>(v);
+    return v;
+}
+
+// Forward substitution of a 16 x 16 unit lower triangular block, columns J ..:
+// ar[i] holds A[i][lane] (lanes 0-15), tc[i] row i of the solution's column
+// `lane`.
+template <int J>
+__device__ __forceinline__ void solve_columns(const float (&ar)[16], float (&tc)[16]) {
+    if constexpr (J < 15) {
+#pragma unroll
+        for (int i = J + 1; i < 16; ++i) tc[i] = fmaf(-dpp_mov<0x150 + J>(ar[i]), tc[J], tc[i]);
+        solve_columns<J + 1>(ar, tc);
+    }
 }
 
 // LDS carve-up of the chunk-local kernel (bytes). T (fp32) reuses the Q
@@ -235,8 +264,8 @@ constexpr int kTile128 = kC * kLD * 2;            // one [64][136] bf16 array
 constexpr int kOffK = 0;                          // K hi, lo
 constexpr int kOffQ = 2 * kTile128;               // Q hi, lo; then T fp32 [2][64][65]
 constexpr int kOffA = 4 * kTile128;               // A fp32 [2][64][65]
-constexpr int kOffS = kOffA + 2 * kC * 65 * 4;    // off-diagonal solve scratch [6][16][17] fp32
-constexpr int kOffG = kOffS + 6 * 16 * 17 * 4;    // G [2][64], beta [2][64]
+constexpr int kOffS = kOffA + 2 * kC * 65 * 4;    // off-diagonal solve scratch [8][16][17] fp32
+constexpr int kOffG = kOffS + 8 * 16 * 17 * 4;    // G [2][64], beta [2][64]
 constexpr int kLocalSmem = kOffG + 4 * kC * 4;
 static_assert(2 * kC * 65 * 4 <= 2 * kTile128, "T must fit the Q region");
 
@@ -252,11 +281,11 @@ static_assert(2 * kC * 65 * 4 <= 2 * kTile128, "T must fit the Q region");
 //       K Q^T (waves 4-7), one query tile each over every key tile, whose
 //       accumulators are P's operand blocks: P of both heads (decay and
 //       mask applied) straight from registers to global; the next unit's
-//       inputs are requested here;
+//       inputs are requested here (waves 4-7: after the next phase);
 //   K image and Q blocks out;
 //   T = (I + A)^-1 of both heads: the eight diagonal blocks by forward
-//       substitution (one wave each), the off-diagonal blocks by six waves
-//       walking their column block down on fp32 MFMAs;
+//       substitution (one wave each), the off-diagonal blocks by halves on
+//       fp32 MFMAs;
 //   T blocks out.
 // Global loads are issued before the stores of the same unit (vmcnt counts
 // stores too on gfx950, so a load consumed after stores would wait for them).
@@ -316,14 +345,9 @@ __global__ __launch_bounds__(kLocalThreads) void dn_chunk_local_kernel(
         const bool ok = lane < nv;
         const float av = hh ? in.av[1] : in.av[0], bv = hh ? in.bv[1] : in.bv[0];
         const float alog = hh ? in.alog[1] : in.alog[0], dtb = hh ? in.dtb[1] : in.dtb[0];
-        float x = ok ? -expf(alog) * softplus(av + dtb) : 0.0f;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const float y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
+        const float x = wave_inclusive_scan(ok ? -expf(alog) * softplus(av + dtb) : 0.0f);
         const float beta = ok ? sigmoid(bv) : 0.0f;
-        const float gc = __shfl(x, 63, 64);
+        const float gc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
         const float eg = __builtin_amdgcn_exp2f(x * kLog2e);
         Gs[hh * kC + lane] = x;
         Bs[hh * kC + lane] = beta;
@@ -399,6 +423,7 @@ __global__ __launch_bounds__(kLocalThreads) void dn_chunk_local_kernel(
     unsigned grabbed = 0;
     if (t == 0) grabbed = atomicAdd(sched, 1u);
     int unn;
+    const bool more = __builtin_amdgcn_readfirstlane(un) < units;   // wave-uniform
 
     // ---- waves 0-3: K K^T -> A of both heads (strictly lower, scaled), row
     // tile rt; waves 4-7: K Q^T for query tile rt over every key tile, whose
@@ -411,10 +436,9 @@ __global__ __launch_bounds__(kLocalThreads) void dn_chunk_local_kernel(
 #pragma unroll
         for (int cj = 0; cj < 4; ++cj) acc[0][cj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         mma_block_x3<128, 1, 4, false>(acc, Kh, Kl, kLD, 16 * rt, Kh, Kl, kLD, 0, lane);
-        // the next unit's inputs (the unit index is clamped, so the loads
-        // stay in bounds when the queue has run out)
+        // the next unit's inputs, if there is one
         unn = s_next;
-        fetch_unit<IN_DT>(in, un < units ? un : u, T, qkv, a, b, a_log, dt_bias, conv_w, wave, lane);
+        if (more) fetch_unit<IN_DT>(in, un, T, qkv, a, b, a_log, dt_bias, conv_w, wave, lane);
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
             const float* G = Gs + hh * kC;
@@ -446,7 +470,6 @@ __global__ __launch_bounds__(kLocalThreads) void dn_chunk_local_kernel(
         for (int kt = 0; kt < 4; ++kt) acc[kt][0] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         mma_block_x3<128, 4, 1, false>(acc, Kh, Kl, kLD, 0, Qh, Ql, kLD, 16 * rt, lane);
         unn = s_next;
-        fetch_unit<IN_DT>(in, un < units ? un : u, T, qkv, a, b, a_log, dt_bias, conv_w, wave, lane);
         const int i = 16 * rt + n;   // this lane's query token
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh) {
@@ -503,50 +526,71 @@ __global__ __launch_bounds__(kLocalThreads) void dn_chunk_local_kernel(
         }
     }
     __syncthreads();   // Q consumed: its region holds T from here on
+    // waves 4-7 request the next unit's inputs here: their P blocks make the
+    // phase above the longer one for them (10-11 thousand cycles against 6-7
+    // of waves 0-3 with the requests in it)
+    if (more && role) fetch_unit<IN_DT>(in, un, T, qkv, a, b, a_log, dt_bias, conv_w, wave, lane);
     // ---- T = (I + A)^-1 (lower unitriangular) in 16x16 blocks, fp32 ------------
     // diagonal block bi of head hh by forward substitution (lanes 0-15, lane =
-    // column), the blocks right of it zeroed by the whole wave
+    // column); the block right of an even one shares its 32-wide k step and is
+    // zeroed by the whole wave
     {
         const int hh = wave >> 2, bi = wave & 3;
         const float* A = Am + hh * kC * 65;
         float* Th = Tm + hh * kC * 65;
-        for (int idx = lane; idx < 16 * (48 - 16 * bi); idx += 64) {
-            const int i = idx / (48 - 16 * bi), j = 16 * (bi + 1) + idx % (48 - 16 * bi);
-            Th[(16 * bi + i) * 65 + j] = 0.0f;
+        if ((bi & 1) == 0) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) Th[(16 * bi + 4 * k + kb) * 65 + 16 * (bi + 1) + n] = 0.0f;
         }
         if (lane < 16) {
-            float tc[16];
+            // column by column: T's row j is final once columns < j are in, and
+            // every later row takes A_ij T_j at once, A_ij broadcast from lane
+            // j of the row the wave holds it in (row_newbcast; the LDS reads of
+            // A all go out ahead of the chain)
+            float ar[16], tc[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                float ac[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int i = 1; i < 16; ++i) ar[i] = A[(16 * bi + i) * 65 + 16 * bi + lane];
 #pragma unroll
-                for (int j = 0; j < i; ++j) ac[j & 3] = fmaf(A[(16 * bi + i) * 65 + 16 * bi + j], tc[j], ac[j & 3]);
-                tc[i] = (i == lane ? 1.0f : 0.0f) - ((ac[0] + ac[1]) + (ac[2] + ac[3]));
-                Th[(16 * bi + i) * 65 + 16 * bi + lane] = tc[i];
-            }
+            for (int i = 0; i < 16; ++i) tc[i] = i == lane ? 1.0f : 0.0f;
+            solve_columns<0>(ar, tc);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) Th[(16 * bi + i) * 65 + 16 * bi + lane] = tc[i];
         }
     }
     __syncthreads();
-    // off-diagonal: T_ij = -T_ii sum_{k=j}^{i-1} A_ik T_kj, wave (hh, bj)
-    // walking column block bj downwards (fp32 MFMA 16x16x4)
-    if (wave < 6) {
-        const int hh = wave / 3, bj = wave % 3;
+    // off-diagonal blocks by halves (fp32 MFMA 16x16x4): T10 = -T11 A10 T00 and
+    // T32 = -T33 A32 T22, then the lower left half -T[23,23] (A[23,01]
+    // T[01,01]), a block per wave each: six products in a chain (a column
+    // block walked down by one wave took nine)
+    {
+        const int hh = wave >> 2, q = wave & 3;
         const float* A = Am + hh * kC * 65;
         float* Th = Tm + hh * kC * 65;
-        float* scr = Scr + wave * (16 * 17);
-        for (int bi = bj + 1; bi < 4; ++bi) {
-            f32x4_t ac = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            for (int bk = bj; bk < bi; ++bk)
-                ac = mm16_f32(A + (16 * bi) * 65 + 16 * bk, 65, Th + (16 * bk) * 65 + 16 * bj, 65, ac, lane);
+        float* const scr = Scr + wave * (16 * 17);
+        const f32x4_t zero = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        auto blk = [](int bi, int bj) { return 16 * bi * 65 + 16 * bj; };
+        auto put = [&](float* dst, int ld, f32x4_t v) {
 #pragma unroll
-            for (int ii = 0; ii < 4; ++ii) scr[(4 * kb + ii) * 17 + n] = ac[ii];
+            for (int ii = 0; ii < 4; ++ii) dst[(4 * kb + ii) * ld + n] = v[ii];
+        };
+        if (q < 2) {   // (2 q + 1, 2 q)
+            put(scr, 17, mm16_f32(A + blk(2 * q + 1, 2 * q), 65, Th + blk(2 * q, 2 * q), 65, zero, lane));
             __builtin_amdgcn_wave_barrier();
-            const f32x4_t res = mm16_f32(Th + (16 * bi) * 65 + 16 * bi, 65, scr, 17,
-                                         f32x4_t{0.f, 0.f, 0.f, 0.f}, lane);
-#pragma unroll
-            for (int ii = 0; ii < 4; ++ii) Th[(16 * bi + 4 * kb + ii) * 65 + 16 * bj + n] = -res[ii];
-            __builtin_amdgcn_wave_barrier();
+            put(Th + blk(2 * q + 1, 2 * q), 65, -mm16_f32(Th + blk(2 * q + 1, 2 * q + 1), 65, scr, 17, zero, lane));
         }
+        __syncthreads();
+        const int bi = 2 + (q >> 1), bj = q & 1;
+        {
+            f32x4_t m = mm16_f32(A + blk(bi, 1), 65, Th + blk(1, bj), 65, zero, lane);
+            if (bj == 0) m = mm16_f32(A + blk(bi, 0), 65, Th + blk(0, 0), 65, m, lane);
+            put(scr, 17, m);
+        }
+        __syncthreads();
+        const float* const m2 = Scr + (4 * hh + bj) * (16 * 17);       // rows of block 2
+        const float* const m3 = Scr + (4 * hh + 2 + bj) * (16 * 17);   // rows of block 3
+        f32x4_t r = mm16_f32(Th + blk(bi, 2), 65, m2, 17, zero, lane);
+        if (bi == 3) r = mm16_f32(Th + blk(3, 3), 65, m3, 17, r, lane);
+        put(Th + blk(bi, bj), 65, -r);
     }
     __syncthreads();
     // ---- T blocks out (bf16 hi / lo) --------------------------------------------
