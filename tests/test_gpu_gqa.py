@@ -223,6 +223,28 @@ def test_gqa_prefill_matches_token_by_token(hip, T, start):
     _prefill_case(hip, T, start, max_ctx=2048, out_dtype=torch.float32 if T == 17 else torch.bfloat16)
 
 
+@pytest.mark.parametrize("kv", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("io", [torch.bfloat16, torch.float32])
+def test_gqa_prefill_rows_do_not_depend_on_the_slice(hip, io, kv):
+    """A 1030-token prompt (three rounds of heads per wave) against its first
+    1000 tokens alone (a round per wave): the same cache rows bit for bit, the
+    same outputs (each row sees the same tiles in the same order)."""
+    import qff
+    print(f"gqa_prefill 1030 / 1000 tokens io={io} kv={kv}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    qg, k, v = (torch.empty(1030, h, d, dtype=io, device=DEV).normal_(generator=g) for h, d in ((16, 512), (2, 256), (2, 256)))
+    p = {n: f32_tensor(w) for n, w in synth.gqa_params().items()}
+    ctx = qff.Context(max_batch=1, max_ctx=1030, max_prefill_tokens=1030)
+    res = []
+    for T in (1030, 1000):
+        kc, vc = (torch.zeros(1030, 2, 256, dtype=kv, device=DEV) for _ in range(2))
+        out = qff.gqa_prefill(ctx, p, qg[:T], k[:T], v[:T], kc, vc, out_dtype=torch.float32)
+        torch.cuda.synchronize()
+        res.append((kc[:1000].view(torch.int16), vc[:1000].view(torch.int16), out[:1000]))
+    for a, b in zip(*res):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("T,start,max_ctx", [(5, 17000, 17024), (33, 511, 576), (250, 256, 512), (40, 1003, 1050)])
 def test_gqa_prefill_in_shares(hip, T, start, max_ctx):
     """Few tokens behind a cache, the tiles shared out over several workgroups
