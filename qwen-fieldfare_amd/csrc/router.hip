@@ -407,20 +407,24 @@ __global__ __launch_bounds__(256) void router_top8_kernel(const float* __restric
 }
 
 // Enough tokens for every CU: a workgroup takes 16 tokens and all experts (wave
-// w experts 32 w .. 32 w + 31, two MFMA tiles over all of K) and ranks its
-// tokens itself. Each slab of 512 columns of x is converted once per
-// workgroup (thread quads, rt_stage_x) into LDS; the weights are requested a
-// slab ahead into registers.
-constexpr int kRtSlab = 8;   // groups per slab
+// w experts 16 w .. 16 w + 15, one MFMA tile over all of K) and ranks its
+// tokens itself, one per wave. Each slab of 512 columns of x is converted
+// once per workgroup (thread quads, rt_stage_x) into LDS; the weights are
+// requested a slab ahead into registers. What bounds it is LDS: every wave
+// reads the slab's x (2 MB a block in all) and turns its weights there (sixteen
+// waves against eight with two tiles each: 57.6 / 60.1 us at 8192 tokens, bf16
+// 45.8 / 49.5).
+constexpr int kRtSlab = 8;          // groups per slab
+constexpr int kRtBlockWaves = 16;
 
-template <int SB_DT, int X_DT, int NW>
-__global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
+template <int SB_DT, int X_DT>
+__global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel(
     const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
     const void* __restrict__ x, float* __restrict__ logits, int32_t* __restrict__ indices,
     float* __restrict__ scores, int experts, int cols, int batch) {
     constexpr bool HILO = X_DT == 0;
-    constexpr int RE = 32 * NW, XL = HILO ? 4 : 2, QT = 8 / NW;   // QT quads (token, group) per thread and slab
-    static_assert(RE == 256, "a workgroup holds every expert");
+    constexpr int NW = kRtBlockWaves, RE = 256, TW = 16 / NW, XL = HILO ? 4 : 2;   // TW tiles of 16 experts per wave
+    constexpr int SBT = RE * kRtSlab / (64 * NW);                                   // scale entries per thread and slab
     constexpr int XS = 16 * 512;                                  // fp16 values of a slab
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int n = lane & 15, kb = lane >> 4;
@@ -429,30 +433,30 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
 
     __shared__ __attribute__((aligned(16))) uint16_t xs[2][HILO ? 2 : 1][XS];
     __shared__ __attribute__((aligned(16))) float sbl[2][kRtSlab * (RE + 2) * 2];
-    __shared__ __attribute__((aligned(16))) uint32_t wl[NW][2][256];   // per wave: a tile's 16 rows x 64 bytes
+    __shared__ __attribute__((aligned(16))) uint32_t wl[NW][TW][256];   // per wave: a tile's 16 rows x 64 bytes
     __shared__ float2 xf[2][kRtSlab][16];   // (sum, 2^e) of (group, token)
 
     // this thread's x quads and scale entries of a slab, and this wave's
     // weights of it: lane (row n, kb) bytes 16 kb .. +15 of each group
-    u32x4_t xr[QT][XL], wr[kRtSlab][2];
-    float sv[4], bv[4];
-    const uint32_t* wrow[2];
+    u32x4_t xr[XL], wr[kRtSlab][TW];
+    float sv[SBT], bv[SBT];
+    // the first eight waves' threads hold a slab's 128 (token, group) quads
+    const bool stager = __builtin_amdgcn_readfirstlane(wave) < 8;   // wave-uniform
+    const uint32_t* wrow[TW];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-        wrow[i] = w + static_cast<size_t>(min(32 * wave + 16 * i + (lane >> 2), experts - 1)) * (cols / 4) + 4 * (lane & 3);
+    for (int i = 0; i < TW; ++i)
+        wrow[i] = w + static_cast<size_t>(min(16 * (TW * wave + i) + (lane >> 2), experts - 1)) * (cols / 4) + 4 * (lane & 3);
     auto fetch_x = [&](int sl) {
+        if (!stager) return;
+        const int q = t >> 2, tok = q >> 3, g = min(kRtSlab * sl + (q & 7), G - 1);
+        const char* src = static_cast<const char*>(x) +
+                          (static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 64 * g) * (HILO ? 4 : 2) + 16 * (t & 3);
 #pragma unroll
-        for (int k = 0; k < QT; ++k) {
-            const int q = (t >> 2) + 16 * NW * k, tok = q >> 3, g = min(kRtSlab * sl + (q & 7), G - 1);
-            const char* src = static_cast<const char*>(x) +
-                              (static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 64 * g) * (HILO ? 4 : 2) + 16 * (t & 3);
-#pragma unroll
-            for (int i = 0; i < XL; ++i) xr[k][i] = *reinterpret_cast<const u32x4_t*>(src + 64 * i);
-        }
+        for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const u32x4_t*>(src + 64 * i);
     };
     auto fetch_sb = [&](int sl) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < SBT; ++k) {
             const int idx = t + 64 * NW * k, e = idx >> 3, g = kRtSlab * sl + (idx & 7);
             const size_t gi = static_cast<size_t>(min(e, experts - 1)) * G + min(g, G - 1);
             sv[k] = elem<SB_DT>::load(scales, gi);
@@ -461,22 +465,21 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
     };
     auto fetch_w = [&](int sl, int gl) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < TW; ++i)
             wr[gl][i] = *reinterpret_cast<const u32x4_t*>(wrow[i] + 16 * min(kRtSlab * sl + gl, G - 1));
     };
     // the fetched slab into LDS buffer buf (groups past the last get zero scales)
     auto stage = [&](int sl, int buf) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < SBT; ++k) {
             const int idx = t + 64 * NW * k, e = idx >> 3, gl = idx & 7;
             const bool live = kRtSlab * sl + gl < G;
             *reinterpret_cast<float2*>(&sbl[buf][(gl * (RE + 2) + e) * 2]) =
                 make_float2(live ? sv[k] : 0.0f, live ? fmaf(128.0f, sv[k], bv[k]) : 0.0f);
         }
-#pragma unroll
-        for (int k = 0; k < QT; ++k) {
-            const int q = (t >> 2) + 16 * NW * k, tok = q >> 3, gl = q & 7, j = t & 3;
-            const float2 xs2 = rt_stage_x<HILO>(xr[k], xs[buf][0], xs[buf][HILO ? 1 : 0], 512, tok, 8 * gl, j);
+        if (stager) {
+            const int q = t >> 2, tok = q >> 3, gl = q & 7, j = t & 3;
+            const float2 xs2 = rt_stage_x<HILO>(xr, xs[buf][0], xs[buf][HILO ? 1 : 0], 512, tok, 8 * gl, j);
             if (j == 0) xf[buf][gl][tok] = xs2;
         }
     };
@@ -488,14 +491,14 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
     // (a clobber after each slab's requests: otherwise the compiler moves the
     // loads to the top of the iteration that uses them)
     asm volatile("" ::: "memory");
-    f32x4_t tot[2];
+    f32x4_t tot[TW];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < TW; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     for (int sl = 0; sl < NS; ++sl) {
         const int buf = sl & 1;
-        f32x4_t acc[2];   // the slab's own sums: shorter fp32 chains
+        f32x4_t acc[TW];   // the slab's own sums: shorter fp32 chains
 #pragma unroll
-        for (int i = 0; i < 2; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TW; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
         stage(sl, buf);
         __syncthreads();
         // the next slab (the last again at the end: no branch around loads)
@@ -513,7 +516,7 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
                 if (HILO) xl[ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][HILO ? 1 : 0][o]);
             }
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < TW; ++i) {
                 const u32x4_t wd = rt_tile_turn(wl[wave][i], wr[gl][i], lane);
                 u32x4_t a[2];
 #pragma unroll
@@ -530,7 +533,7 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
                 }
                 P = mfma_16x16x32_f16(a[0], xh[0], P);
                 P = mfma_16x16x32_f16(a[1], xh[1], P);
-                const f32x4_t* sb = reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 32 * wave + 16 * i + 4 * kb) * 2]);
+                const f32x4_t* sb = reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 16 * (TW * wave + i) + 4 * kb) * 2]);
                 const f32x4_t c0 = sb[0], c1 = sb[1];
                 acc[i][0] = fmaf(c0[0], P[0] * sf.y, fmaf(c0[1], sf.x, acc[i][0]));
                 acc[i][1] = fmaf(c0[2], P[1] * sf.y, fmaf(c0[3], sf.x, acc[i][1]));
@@ -540,7 +543,7 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
             fetch_w(nx, gl);
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) tot[i] += acc[i];
+        for (int i = 0; i < TW; ++i) tot[i] += acc[i];
         asm volatile("" ::: "memory");
     }
     // lane: token n, experts 32 wave + 16 i + 4 kb .. +3
@@ -549,8 +552,8 @@ __global__ __launch_bounds__(64 * NW) void router_logits_block_kernel(
     __syncthreads();
     float* lg = reinterpret_cast<float*>(xs);   // [16][RE + 4]
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-        *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 32 * wave + 16 * i + 4 * kb]) = tot[i];
+    for (int i = 0; i < TW; ++i)
+        *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 16 * (TW * wave + i) + 4 * kb]) = tot[i];
     __syncthreads();
     for (int tok = wave; tok < 16; tok += NW) {
         const int m = M0 + tok;
@@ -602,7 +605,7 @@ hipError_t launch_router_top8(qff_ctx* ctx, hipStream_t stream, const uint32_t* 
     //   MFMA, 1 tile    158 / 46.4 / 17.8 / 11.2 (bf16 x at 16: 10.1)
     //   MFMA, 2 tiles    92 / 31.8 / 14.5 / 12.4
     //   MFMA, 4 tiles    77 / 26.4 / 17.7 / 16.6
-    //   whole blocks     61 / 29.3 / 27.7 / 26.4 (33 against 44.5 at 4096)
+    //   whole blocks     58 / 28.4 / 26.4 / 26.0 (32 against 44.5 at 4096)
     // so the tiles per workgroup grow once the grid covers the chip, and whole
     // blocks take over where they do so themselves.
     const int nb = (batch + 15) / 16, cu = ctx->num_cu;
@@ -610,7 +613,8 @@ hipError_t launch_router_top8(qff_ctx* ctx, hipStream_t stream, const uint32_t* 
     if (8 * nb > 5 * cu) {
         ProfScope prof(ctx, stream, "router_logits");
 #define QFF_RB(S, X) \
-    router_logits_block_kernel<S, X, 8><<<nb, 512, 0, stream>>>(w, s, b, x, logits, indices, scores, experts, cols, batch)
+    router_logits_block_kernel<S, X><<<nb, 64 * kRtBlockWaves, 0, stream>>>(w, s, b, x, logits, indices, scores, experts, \
+                                                                           cols, batch)
         if (sb_dtype == QFF_BF16) {
             if (x_dtype == QFF_BF16) QFF_RB(1, 1); else QFF_RB(1, 0);
         } else {
