@@ -41,7 +41,9 @@ struct qff_ctx {
     uint16_t* gqa_kv16 = nullptr;   // fp16 copy of a bf16 K cache for prefill: [max_ctx][2][256]
     uint16_t* gqa_vt = nullptr;     // transposed fp16 copy of the V cache for prefill: [2][max_ctx / 64][256][64]
     // Many-token Q4 products, per slice of q4_xs_tokens tokens: the fp16
-    // activations x16 [q4_xs_tokens][<= 4096] and each token's output factor.
+    // activations x16 (q4_xs_tokens rounded up to 32, <= 4096 columns; row or
+    // MFMA operand order by the kernel that reads them) and each token's output
+    // factor.
     uint16_t* q4_x16 = nullptr;
     float* q4_fm = nullptr;
     int q4_xs_tokens = 0;

@@ -954,11 +954,15 @@ __global__ __launch_bounds__(64 * kQ4VecWaves) void q4_gemv1_kernel(Q4Parts part
 constexpr int kQ4GemmRows = 256;   // weight rows per workgroup
 constexpr int kQ4GemmToks = 128;   // tokens per workgroup
 
-// x16 lies in the order of the 32x32x16 MFMA's B operand: per token tile of 32,
+// For q4_gemm_split_kernel x16 lies in the order of the 32x32x16 MFMA's B operand:
+// per token tile of 32,
 // group of 64 columns and step ks a block of 64 lanes x 16 bytes, lane 32 h + r
 // holding token r's 8-column piece 4 h + ks of the group, so an operand is one
 // contiguous 1-KB read (a lane per token row costs the load unit four times
-// as many cycles). `piece` is the token's 8-column block over the row.
+// as many cycles). `piece` is the token's 8-column block over the row. For
+// q4_gemm_kernel, whose staging copies reach LDS from any order, x16 is
+// [tokens][cols]: in the operand order this pass took 0.7-1 us more and that
+// kernel up to 2 (in-projection of 12352 rows at 2000 tokens 148 against 144.6).
 __device__ __forceinline__ size_t q4_x16_at(int m, int piece, int G) {
     const int g = piece >> 3, h = (piece >> 2) & 1, ks = piece & 3;
     return ((static_cast<size_t>(m >> 5) * G + g) * 4 + ks) * 512 + (32 * h + (m & 31)) * 8;
@@ -967,8 +971,8 @@ __device__ __forceinline__ size_t q4_x16_at(int m, int piece, int G) {
 // x16 and f_m, WPT waves per token: thread i of a token's 64 WPT holds 8-column
 // blocks i, i + 64 WPT, .. One wave per token (TPB tokens a workgroup) where
 // the tokens fill the chip; four for short batches, whose time is one wave's
-// chain of loads, maxima and stores.
-template <int X_DT, bool NORM, int WPT, int TPB>
+// chain of loads, maxima and stores. ROWS: x16 as [tokens][cols].
+template <int X_DT, bool NORM, int WPT, int TPB, bool ROWS>
 __global__ __launch_bounds__(64 * WPT * TPB) void q4_x16_kernel(const void* __restrict__ x, uint16_t* __restrict__ x16,
                                                      float* __restrict__ fm, int cols, int batch, Q4Norm nrm) {
     static_assert(WPT == 1 || TPB == 1, "several waves a token, or several tokens a workgroup");
@@ -1033,14 +1037,16 @@ __global__ __launch_bounds__(64 * WPT * TPB) void q4_x16_kernel(const void* __re
     // TPB tokens meet in LDS per 64 blocks, so that TPB lanes write 16 TPB
     // consecutive bytes (a lane per block writes 64 separate lines an
     // instruction: 14 us more at 8192 x 4096)
-    __shared__ u32x4_t xo[TPB > 1 ? 2 : 1][TPB > 1 ? 64 * (TPB + 1) : 1];
+    __shared__ u32x4_t xo[TPB > 1 && !ROWS ? 2 : 1][TPB > 1 && !ROWS ? 64 * (TPB + 1) : 1];
 #pragma unroll
     for (int i = 0; i < kMaxB; ++i) {
         const int b = i0 + 64 * WPT * i;
-        if (TPB == 1 && b >= nb) break;
+        if ((TPB == 1 || ROWS) && b >= nb) break;
         const u32x4_t h{pack_f16x2(v[i][0] * p, v[i][4] * p), pack_f16x2(v[i][1] * p, v[i][5] * p),
                         pack_f16x2(v[i][2] * p, v[i][6] * p), pack_f16x2(v[i][3] * p, v[i][7] * p)};
-        if constexpr (TPB == 1) {
+        if constexpr (ROWS) {
+            if (mt < batch) *reinterpret_cast<u32x4_t*>(x16 + static_cast<size_t>(m) * cols + 8 * b) = h;
+        } else if constexpr (TPB == 1) {
             *reinterpret_cast<u32x4_t*>(x16 + q4_x16_at(mt, b, G)) = h;
         } else {
             if (64 * i >= nb) break;   // workgroup-uniform
@@ -1104,10 +1110,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         sbl[g * kQ4GemmRows + r] = pack_f16x2(256.0f * elem<SB_DT>::load(scales, gi), 256.0f * elem<SB_DT>::load(biases, gi));
     }
 
-    // x16 staging straight from global memory into LDS: wave w copies the four
-    // operand blocks (steps ks) of token tile w of the group, lane order kept
-    const int xtile = min(M0 / 32 + wave, (batch - 1) / 32);
-    const uint16_t* xsrc = x16 + static_cast<size_t>(xtile) * G * 2048 + 8 * lane;
+    // x16 staging straight from global memory into LDS: wave w's load i fills
+    // tokens 8 (4w + i) .. +7 of the [128][64] tile, lane l the 16-byte
+    // piece l & 7 of token l >> 3, which holds the token's 8-column block
+    // (l & 7) ^ ((token >> 1) & 7) of the group (the swizzle spreads the 32
+    // rows of an operand read over the bank groups)
+    const uint16_t* xsrc[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int tok = 8 * (4 * wave + i) + (lane >> 3);
+        xsrc[i] = x16 + static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 8 * ((lane & 7) ^ ((tok >> 1) & 7));
+    }
     // weight words: lane -> rows 64 wave + 32 rt + r, words 4h .. 4h + 3 of each group
     // (rows past the part's end read its last row; their outputs are not stored)
     const int r = lane & 31, h = lane >> 5;
@@ -1119,8 +1132,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     auto stage_x = [&](int buf, int g) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc + 2048 * g + 512 * i),
-                                             (__attribute__((address_space(3))) void*)&Xl[buf][512 * (4 * wave + i)],
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(xsrc[i] + 64 * g),
+                                             (__attribute__((address_space(3))) void*)&Xl[buf][8 * (4 * wave + i) * 64],
                                              16, 0, 0);
     };
     auto fetch_w = [&](u32x4_t (&dst)[2], int g) {
@@ -1158,7 +1171,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         uint32_t sb[2];
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt) sb[rt] = sbl[g * kQ4GemmRows + 64 * wave + 32 * rt + r];
-        const uint16_t* xb = &Xl[g & 1][8 * lane];   // B operand of token tile mt, step ks: block 4 mt + ks
+        // B operand of token tile mt, step ks: token 32 mt + r, x16 piece
+        // 4h + ks (swizzled by (token / 2) % 8, so the 32 rows of a read
+        // meet every bank group twice)
+        const uint16_t* xb = &Xl[g & 1][r * 64];
+        const int sw = (r >> 1) & 7;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             u32x4_t A[2], B[4];
@@ -1166,7 +1183,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
             for (int rt = 0; rt < 2; ++rt) A[rt] = q4_to_f16_scaled(cur[rt][ks], sb[rt], e1024);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt)
-                B[mt] = *reinterpret_cast<const u32x4_t*>(xb + 512 * (4 * mt + ks));
+                B[mt] = *reinterpret_cast<const u32x4_t*>(xb + 32 * mt * 64 + 8 * ((4 * h + ks) ^ sw));
 #pragma unroll
             for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
@@ -1476,6 +1493,27 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
     const int lds = G * kQ4GemmRows * 4;   // packed (s, b) of the row tile
     QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<1>>(lds)));
     QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<2>>(lds)));
+    // Which kernel: by the tokens and columns alone, and K always split in
+    // four, so that a part's sums do not depend on the rows beside it
+    // (scales and biases are read two groups at a time: an even number of
+    // groups, 4-byte-aligned scale rows). Which tile: the largest that
+    // still covers the chip. fp32 x, x16 pass included, us at 64 / 200 /
+    // 448 / 512 / 1000 / 4096 tokens:
+    //   2048 x 4096, 256 x 128 tiles    73 / 97 / - / 99 / 99 / 149
+    //     K split 32 x 32               12 / 18 / - / 29 / 51
+    //     K split 32 x 64               13 / 17 / - / 25 / 43 / 154
+    //     K split 64 x 64               17 / 21 / - / 25 / 37 / 123
+    //   12352 x 2048, 256 x 128 tiles   45 / 50 / 52.5 / 51 / 78 / 263
+    //     K split 32 x 64               15 / 34 / - / 61
+    //     K split 64 x 64               15 / 33 / 50.5 / 56 / 100
+    //   9216 x 2048, 256 x 128 tiles    - / - / 51 / 51
+    //     K split 64 x 64               - / - / 35.5 / 41
+    // The widest in-projection sets the line at 2048 columns. The large tile
+    // stages the scales of all of K in LDS and so runs one workgroup a CU
+    // above that: it takes over later there.
+    bool split = (cols / 64) % 2 == 0 && batch <= (cols > 2048 ? 4096 : 448);
+    for (int i = 0; i < nparts; ++i)
+        split = split && ((reinterpret_cast<uintptr_t>(parts[i].scales) | reinterpret_cast<uintptr_t>(parts[i].biases)) & 3) == 0;
     for (int m0 = 0; m0 < batch; m0 += ctx->q4_xs_tokens) {
         const int mb = min(ctx->q4_xs_tokens, batch - m0);
         const void* xm = static_cast<const char*>(x) + static_cast<size_t>(m0) * cols * (x_dtype == QFF_BF16 ? 2 : 4);
@@ -1485,8 +1523,9 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
             // launches: 11.3 against 12.3 us at 33, 16.4 / 17.3 at 200; equal at
             // 768, 140 / 131 at 4096)
 #define QFF_X16(X)                                                                                                       \
-    if (mb < 768) q4_x16_kernel<X, NORM, 4, 1><<<mb, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);     \
-    else q4_x16_kernel<X, NORM, 1, 8><<<(mb + 7) / 8, 512, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm)
+    if (!split) q4_x16_kernel<X, NORM, 1, 4, true><<<(mb + 3) / 4, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);     \
+    else if (mb < 768) q4_x16_kernel<X, NORM, 4, 1, false><<<mb, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);      \
+    else q4_x16_kernel<X, NORM, 1, 8, false><<<(mb + 7) / 8, 512, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm)
             if (x_dtype == QFF_BF16) { QFF_X16(1); } else { QFF_X16(0); }
 #undef QFF_X16
         }
@@ -1504,28 +1543,9 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
             return dim3(tiles, (mb + tpb - 1) / tpb);
         };
         const auto count = [](dim3 g) { return static_cast<int>(g.x * g.y); };
-        // Which kernel: by the tokens and columns alone, and K always split in
-        // four, so that a part's sums do not depend on the rows beside it
-        // (scales and biases are read two groups at a time: an even number of
-        // groups, 4-byte-aligned scale rows). Which tile: the largest that
-        // still covers the chip. fp32 x, x16 pass included, us at 64 / 200 /
-        // 512 / 1000 / 4096 tokens:
-        //   2048 x 4096, 256 x 128 tiles    73 / 97 / 99 / 99 / 152
-        //     K split 32 x 32               12 / 18 / 29 / 51
-        //     K split 32 x 64               13 / 17 / 25 / 43 / 154
-        //     K split 64 x 64               17 / 21 / 25 / 37 / 128
-        //   12352 x 2048, 256 x 128 tiles   45 / 50 / 53 / 79 / 260
-        //     K split 32 x 64               15 / 34 / 61
-        //     K split 64 x 64               15 / 33 / 57 / 100
-        // The large tile stages the scales of all of K in LDS and so runs one
-        // workgroup a CU above 2048 columns: it takes over later there.
         Q4Parts P;
         ProfScope prof(ctx, stream, "q4_gemm");
         const int cu = ctx->num_cu, pm = (1 << 20) / std::max(G / 2, 1) + 1;   // idx / (G / 2) = idx pm >> 20, idx < 2048
-        bool split = G % 2 == 0;
-        for (int i = 0; i < nparts; ++i)
-            split = split && ((reinterpret_cast<uintptr_t>(sl[i].scales) | reinterpret_cast<uintptr_t>(sl[i].biases)) & 3) == 0;
-        split = split && batch <= (cols > 2048 ? 4096 : 512);
         dim3 grid;
 #define QFF_SPLIT(RT, MT, WK, D)                                                                               \
     if (sb_dtype == QFF_BF16)                                                                                  \

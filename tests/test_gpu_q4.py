@@ -326,7 +326,8 @@ def test_q4_matmul_parts_4096_cols_f32_x_residual(hip, batch):
 
 @pytest.mark.parametrize("batch,cols,odd", [
     (33, 128, False), (64, 4096, False), (65, 2048, False),     # one pair of groups; whole and ragged token tiles
-    (200, 1152, False), (512, 2048, False), (513, 2048, False),  # the last batch of the split kernel and the next
+    (200, 1152, False), (448, 2048, False), (449, 2048, False),  # the last batch of the split kernel and the next
+    (512, 2048, False), (513, 2048, False),
     (70, 2048, True), (40, 192, False),                          # odd scale addresses; an odd number of groups
     (800, 4096, False),                                          # eight tokens a workgroup in the fp16 pass
 ])
