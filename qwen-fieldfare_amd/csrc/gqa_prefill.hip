@@ -4,8 +4,9 @@
 // The reference has no prefill kernel: each prompt token runs the decode
 // path at its position (QwenQ4ActiveExpertStreamingRunner.swift:1545-1561,
 // 1076-1150), so token t attends to positions 0 .. start+t. This file
-// computes all T rows in two launches:
-//   prep   one wave per token: head RMSNorm + partial RoPE of the
+// computes all T rows in two launches (three where the tiles are shared out,
+// see gqa_prefill_attn_kernel):
+//   prep   one wave per token (three up to 1024 tokens): head RMSNorm + partial RoPE of the
 //          16 q heads (fp16, softmax scale folded in, to workspace: the
 //          reference also rounds q to half, Runner:1119-1126) and of the 2 k
 //          heads (appended to the cache, bf16 or fp16, together with v; a
