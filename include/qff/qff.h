@@ -190,9 +190,9 @@ int qff_q8_dequant(qff_ctx* ctx, qff_stream_t stream, const uint32_t* w,
 /* The MoE router of `batch` tokens: logits[m, e] = sum_c W[e, c] x[m, c]
  * with W [experts, cols] affine-Q8 as above, accumulated in fp32 in the
  * factored form scale * sum(q x) + bias * sum(x) per group (several tokens:
- * over q - 128 with the bias adjusted, x as an fp16 hi + lo pair of at least
- * 22 bits); then per token
- * the eight largest logits in descending order (equal logits: lower expert
+ * over q - 128 with the bias adjusted, an fp32 x as three bf16 terms that hold
+ * every bit of |x| >= 2^-110; so a token's logits can differ in the last bits
+ * between batch sizes); then per token the eight largest logits in descending order (equal logits: lower expert
  * index first) into indices [batch, 8], and their routing weights into
  * scores [batch, 8]: softmax over all `experts` logits shifted by the
  * largest, the eight probabilities divided by their sum. x [batch, cols] of

@@ -21,13 +21,16 @@
 //       loads are issued together and the logits stored at the end (a store
 //       between tokens would hold the next token's loads: vmcnt counts
 //       stores too).
-//   router_logits_mfma_kernel  several tokens, as matrix products: the bytes
-//       become the exact fp16 integers q - 128, x the fp16 pair hi + lo of
-//       x 2^-e with e per (token, group) (22 bits; a bf16 x is exact in hi),
-//       and per group logit += s 2^e P + (b + 128 s) sum(x) in fp32. The
-//       products are exact and a stored scale of ~-128 times the bias no
-//       longer cancels, so the logits are closer to the fp64 product than
-//       the vector form's (1.1e-7 against 2.5e-7 relative). NW waves split K.
+//   router_logits_mfma_kernel  several tokens, as matrix products on bf16
+//       operands: the bytes become the integers q - 128, an fp32 x three
+//       terms that add up to it bit for bit, a bf16 x stays as it is, and per
+//       group logit += s P + (b + 128 s) sum(x) in fp32. The products are
+//       exact and a stored bias of ~-128 times the scale no longer cancels,
+//       so the logits are closer to the fp64 product than the vector form's
+//       (2000 tokens of fp32 x, 2-norm: 0.92e-7 against 2.5e-7; bf16 x 0.81e-7
+//       against 0.91e-7). x as an fp16 hi + lo pair (22 bits) took two thirds
+//       of the products and 1.05e-7: 25.6 us at 2000 tokens either way, 54.6
+//       against 64 at 8192. NW waves split K.
 //       What bounded the first form of it, at 25-30 us a block, was the
 //       operand order itself: a lane per matrix row makes a 16-byte load
 //       touch 64 different lines (38 B/ns per CU from L2 against 125-148
@@ -132,74 +135,94 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint32_t* __re
     }
 }
 
-// Several tokens. grid (ceil(E / (16 NT)), ceil(batch / 16)), NW waves.
-typedef _Float16 rt_f16x2_t __attribute__((ext_vector_type(2)));
+// bf16 operands that hold an x of type X_DT
+template <int X_DT> constexpr int rt_terms = X_DT == 1 ? 1 : 3;
 
-// 4 weight bytes -> the fp16 pairs q - 128 (exact): byte b under the exponent
-// byte 0x64 is the fp16 1024 + b, minus 1152
-__device__ __forceinline__ void rt_bytes_to_f16(uint32_t w, uint32_t& lo, uint32_t& hi) {
-    const rt_f16x2_t k = {static_cast<_Float16>(1152.0f), static_cast<_Float16>(1152.0f)};
-    lo = __builtin_bit_cast(uint32_t, __builtin_bit_cast(rt_f16x2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)) - k);
-    hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(rt_f16x2_t, __builtin_amdgcn_perm(0x64646464u, w, 0x04030402u)) - k);
+// 4 weight bytes -> the bf16 pairs q - 128: integers of at most 8 bits, whose
+// fp32 form has them in its upper half
+__device__ __forceinline__ void rt_bytes_to_bf16(uint32_t w, uint32_t& lo, uint32_t& hi) {
+    const uint32_t v = w ^ 0x80808080u;   // q - 128 as signed bytes
+    uint32_t f[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        f[c] = __float_as_uint(static_cast<float>(static_cast<int8_t>(static_cast<uint8_t>(v >> (8 * c)))));
+    lo = __builtin_amdgcn_perm(f[1], f[0], 0x07060302u);
+    hi = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
 }
 
 // One group (64 columns) of one token, held by the four lanes j of a quad (fp32:
-// columns 16 i + 4 j .. +3 in piece i; bf16: 32 i + 8 j .. +7), as fp16 operands
-// x 2^-e with the group's largest magnitude in [2^13, 2^14) (e >= -127: 2^-e
-// stays finite), hi + lo for fp32 (22 bits; bf16 is exact in hi), into the LDS
-// rows hi, lo [token][row] at 16-byte pieces p0 + c, swizzled by the token.
-// Returns (sum of x, 2^e).
-template <bool HILO, int XL>
-__device__ __forceinline__ float2 rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* hi, uint16_t* lo, int row, int tok,
-                                             int p0, int j) {
-    float v[16];
-#pragma unroll
-    for (int i = 0; i < XL; ++i)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (HILO) {
-                v[4 * i + c] = __uint_as_float(xr[i][c]);
-            } else {
-                v[8 * i + 2 * c] = __uint_as_float(xr[i][c] << 16);
-                v[8 * i + 2 * c + 1] = __uint_as_float(xr[i][c] & 0xffff0000u);
-            }
-        }
-    float sum = 0.0f, mx = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        sum += v[i];
-        mx = fmaxf(mx, fabsf(v[i]));
-    }
-    sum = group_sum<4>(sum);
-    mx = group_max<4>(mx);
-    const int e = mx > 0.0f ? max(__builtin_amdgcn_frexp_expf(mx) - 14, -127) : 0;
-    const float p = ldexpf(1.0f, -e);
+// columns 16 i + 4 j .. +3 in piece i; bf16: 32 i + 8 j .. +7), as bf16
+// operands: a bf16 x as it is, an fp32 x as the three terms that cutting 8
+// significant bits off at a time leaves, hi + mid + lo == x with every bit (of
+// |x| >= 2^-110: below that the last term meets bf16's smallest step, 2^-133).
+// Term k goes to xo[k], LDS rows [token][row] at 16-byte pieces p0 + c,
+// swizzled by the token. Returns the sum of x.
+template <int X_DT, int XL>
+__device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* const (&xo)[rt_terms<X_DT>], int row,
+                                            int tok, int p0, int j) {
     const int sw = tok & (row / 8 - 1) & 15;
-    if (HILO) {
+    float sum = 0.0f;
+    if constexpr (X_DT == 1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            u32x2_t h2, l2;
+        for (int i = 0; i < 2; ++i) {
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                uint32_t hh, ll;
-                split_f16x2(v[4 * i + 2 * c] * p, v[4 * i + 2 * c + 1] * p, hh, ll);
-                h2[c] = hh;
-                l2[c] = ll;
+            for (int c = 0; c < 4; ++c) {
+                sum += __uint_as_float(xr[i][c] << 16);
+                sum += __uint_as_float(xr[i][c] & 0xffff0000u);
             }
-            const int o = tok * row + 8 * ((p0 + 2 * i + (j >> 1)) ^ sw) + 4 * (j & 1);
-            *reinterpret_cast<u32x2_t*>(hi + o) = h2;
-            *reinterpret_cast<u32x2_t*>(lo + o) = l2;
+            *reinterpret_cast<u32x4_t*>(xo[0] + tok * row + 8 * ((p0 + 4 * i + j) ^ sw)) = xr[i];
         }
     } else {
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            u32x4_t h4;
+        for (int i = 0; i < 4; ++i) {
+            uint32_t f[3][4];   // fp32 forms of the terms: the upper halves hold them
 #pragma unroll
-            for (int c = 0; c < 4; ++c) h4[c] = pack_f16x2(v[8 * i + 2 * c] * p, v[8 * i + 2 * c + 1] * p);
-            *reinterpret_cast<u32x4_t*>(hi + tok * row + 8 * ((p0 + 4 * i + j) ^ sw)) = h4;
+            for (int c = 0; c < 4; ++c) {
+                const float v = __uint_as_float(xr[i][c]);
+                sum += v;
+                f[0][c] = xr[i][c];
+                const float r1 = v - __uint_as_float(f[0][c] & 0xffff0000u);
+                f[1][c] = __float_as_uint(r1);
+                f[2][c] = __float_as_uint(r1 - __uint_as_float(f[1][c] & 0xffff0000u));
+            }
+            const int o = tok * row + 8 * ((p0 + 2 * i + (j >> 1)) ^ sw) + 4 * (j & 1);
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+                *reinterpret_cast<u32x2_t*>(xo[k] + o) = u32x2_t{__builtin_amdgcn_perm(f[k][1], f[k][0], 0x07060302u),
+                                                                 __builtin_amdgcn_perm(f[k][3], f[k][2], 0x07060302u)};
         }
     }
-    return make_float2(sum, ldexpf(1.0f, e));
+    return group_sum<4>(sum);
+}
+
+// sum over one group of (q - 128) x for 16 experts (weight bytes wd in operand
+// order) x 16 tokens, the smallest terms of x first
+template <int TERMS>
+__device__ __forceinline__ f32x4_t rt_products(u32x4_t wd, const u32x4_t (&xo)[TERMS][2]) {
+    u32x4_t a[2];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+        uint32_t lo, hi;
+        rt_bytes_to_bf16(wd[d], lo, hi);
+        a[d >> 1][2 * (d & 1)] = lo;
+        a[d >> 1][2 * (d & 1) + 1] = hi;
+    }
+    f32x4_t P = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = TERMS - 1; k >= 0; --k) {
+        P = mfma_16x16x32_bf16(a[0], xo[k][0], P);
+        P = mfma_16x16x32_bf16(a[1], xo[k][1], P);
+    }
+    return P;
+}
+
+// acc += s P + (b + 128 s) sum(x) for the lane's four experts, sb their (s, b + 128 s)
+__device__ __forceinline__ void rt_accumulate(f32x4_t& acc, f32x4_t P, float sum, const f32x4_t* sb) {
+    const f32x4_t c0 = sb[0], c1 = sb[1];
+    acc[0] = fmaf(c0[0], P[0], fmaf(c0[1], sum, acc[0]));
+    acc[1] = fmaf(c0[2], P[1], fmaf(c0[3], sum, acc[1]));
+    acc[2] = fmaf(c1[0], P[2], fmaf(c1[1], sum, acc[2]));
+    acc[3] = fmaf(c1[2], P[3], fmaf(c1[3], sum, acc[3]));
 }
 
 // A 16-row x 64-byte tile from the load's lane order (lane l: row l / 4, piece
@@ -215,6 +238,7 @@ __device__ __forceinline__ u32x4_t rt_tile_turn(uint32_t* buf, u32x4_t v, int la
     return o;
 }
 
+// Several tokens. grid (ceil(E / (16 NT)), ceil(batch / 16)), NW waves.
 template <int SB_DT, int X_DT, int NT, int NW>
 __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint32_t* __restrict__ w,
                                                                      const uint16_t* __restrict__ scales,
@@ -222,9 +246,9 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
                                                                      const void* __restrict__ x,
                                                                      float* __restrict__ logits, int experts, int cols,
                                                                      int batch, int gmagic) {
-    constexpr bool HILO = X_DT == 0;   // fp32 x: hi + lo operands; bf16 x is exact in hi
-    constexpr int RE = 16 * NT;        // experts per workgroup
-    constexpr int XL = HILO ? 4 : 2;   // 16-byte x loads per lane and group
+    constexpr int TERMS = rt_terms<X_DT>, XB = X_DT == 1 ? 2 : 4;   // operands and bytes of an x
+    constexpr int RE = 16 * NT;   // experts per workgroup
+    constexpr int XL = XB;        // 16-byte x loads per lane and group
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int n = lane & 15, kb = lane >> 4;
     const int G = cols / 64;
@@ -232,13 +256,13 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
     // (s, b + 128 s) of the workgroup's experts, [G][RE]; afterwards the waves' partial logits [NW][RE x 16]
     constexpr int kSb = 64 * (RE + 2) * 2, kPart = NW * RE * 16;
     __shared__ __attribute__((aligned(16))) float lds[kSb > kPart ? kSb : kPart];
-    // per wave: a weight tile, the group's x (hi, lo) [16 tokens][64] and each token's (sum, 2^e)
+    // per wave: a weight tile, the group's x operands [16 tokens][64] and each token's sum
     __shared__ __attribute__((aligned(16))) uint32_t wl[NW][256];
-    __shared__ __attribute__((aligned(16))) uint16_t xl[NW][HILO ? 2 : 1][16 * 64];
-    __shared__ float2 xf[NW][16];
+    __shared__ __attribute__((aligned(16))) uint16_t xl[NW][TERMS][16 * 64];
+    __shared__ float xf[NW][16];
 
     const char* xrow = static_cast<const char*>(x) +
-                       static_cast<size_t>(min(M0 + (lane >> 2), batch - 1)) * cols * (HILO ? 4 : 2) + 16 * (lane & 3);
+                       static_cast<size_t>(min(M0 + (lane >> 2), batch - 1)) * cols * XB + 16 * (lane & 3);
     const uint32_t* wrow[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i)
@@ -246,7 +270,7 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
 
     u32x4_t xr[2][XL], wr[2][NT];
     auto fetch = [&](int s, int g) {
-        const char* xp = xrow + 64 * g * (HILO ? 4 : 2);
+        const char* xp = xrow + 64 * g * XB;
 #pragma unroll
         for (int q = 0; q < XL; ++q) xr[s][q] = *reinterpret_cast<const u32x4_t*>(xp + 64 * q);
 #pragma unroll
@@ -277,42 +301,25 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
 #pragma unroll
     for (int i = 0; i < NT; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     auto step = [&](int s, int g) {
-        const float2 xs = rt_stage_x<HILO>(xr[s], xl[wave][0], xl[wave][HILO ? 1 : 0], 64, lane >> 2, 0, lane & 3);
+        uint16_t* xo[TERMS];
+#pragma unroll
+        for (int k = 0; k < TERMS; ++k) xo[k] = xl[wave][k];
+        const float xs = rt_stage_x<X_DT>(xr[s], xo, 64, lane >> 2, 0, lane & 3);
         if ((lane & 3) == 0) xf[wave][lane >> 2] = xs;
         __builtin_amdgcn_wave_barrier();
-        const float2 sf = xf[wave][n];
-        u32x4_t xh[2], xw[2];
+        const float sum = xf[wave][n];
+        u32x4_t xv[TERMS][2];
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) {
             const int o = n * 64 + 8 * ((2 * kb + ks) ^ (n & 7));
-            xh[ks] = *reinterpret_cast<const u32x4_t*>(&xl[wave][0][o]);
-            if (HILO) xw[ks] = *reinterpret_cast<const u32x4_t*>(&xl[wave][HILO ? 1 : 0][o]);
+#pragma unroll
+            for (int k = 0; k < TERMS; ++k) xv[k][ks] = *reinterpret_cast<const u32x4_t*>(&xl[wave][k][o]);
         }
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
-            const u32x4_t wd = rt_tile_turn(wl[wave], wr[s][i], lane);
-            u32x4_t a[2];
-#pragma unroll
-            for (int d = 0; d < 4; ++d) {
-                uint32_t lo, hi;
-                rt_bytes_to_f16(wd[d], lo, hi);
-                a[d >> 1][2 * (d & 1)] = lo;
-                a[d >> 1][2 * (d & 1) + 1] = hi;
-            }
-            f32x4_t P = f32x4_t{0.f, 0.f, 0.f, 0.f};
-            if (HILO) {
-                P = mfma_16x16x32_f16(a[0], xw[0], P);
-                P = mfma_16x16x32_f16(a[1], xw[1], P);
-            }
-            P = mfma_16x16x32_f16(a[0], xh[0], P);
-            P = mfma_16x16x32_f16(a[1], xh[1], P);
+            const f32x4_t P = rt_products<TERMS>(rt_tile_turn(wl[wave], wr[s][i], lane), xv);
             // experts 16 i + 4 kb .. +3
-            const f32x4_t* sb = reinterpret_cast<const f32x4_t*>(&lds[(g * (RE + 2) + 16 * i + 4 * kb) * 2]);
-            const f32x4_t c0 = sb[0], c1 = sb[1];
-            acc[i][0] = fmaf(c0[0], P[0] * sf.y, fmaf(c0[1], sf.x, acc[i][0]));
-            acc[i][1] = fmaf(c0[2], P[1] * sf.y, fmaf(c0[3], sf.x, acc[i][1]));
-            acc[i][2] = fmaf(c1[0], P[2] * sf.y, fmaf(c1[1], sf.x, acc[i][2]));
-            acc[i][3] = fmaf(c1[2], P[3] * sf.y, fmaf(c1[3], sf.x, acc[i][3]));
+            rt_accumulate(acc[i], P, sum, reinterpret_cast<const f32x4_t*>(&lds[(g * (RE + 2) + 16 * i + 4 * kb) * 2]));
         }
         __builtin_amdgcn_wave_barrier();
     };
@@ -410,10 +417,10 @@ __global__ __launch_bounds__(256) void router_top8_kernel(const float* __restric
 // w experts 16 w .. 16 w + 15, one MFMA tile over all of K) and ranks its
 // tokens itself, one per wave. Each slab of 512 columns of x is converted
 // once per workgroup (thread quads, rt_stage_x) into LDS; the weights are
-// requested a slab ahead into registers. What bounds it is LDS: every wave
-// reads the slab's x (2 MB a block in all) and turns its weights there (sixteen
-// waves against eight with two tiles each: 57.6 / 60.1 us at 8192 tokens, bf16
-// 45.8 / 49.5).
+// requested a slab ahead into registers. What seems to bound it is LDS: every
+// wave reads the slab's x (3 MB a block in all, 1 MB of bf16) and turns its
+// weights there (sixteen waves against eight with two tiles each: 64.1 / 65.9
+// us at 8192 tokens, 58.3 / 63.1 at 5000, bf16 46.6 / 51.4 at 8192).
 constexpr int kRtSlab = 8;          // groups per slab
 constexpr int kRtBlockWaves = 16;
 
@@ -422,19 +429,19 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     const uint32_t* __restrict__ w, const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
     const void* __restrict__ x, float* __restrict__ logits, int32_t* __restrict__ indices,
     float* __restrict__ scores, int experts, int cols, int batch) {
-    constexpr bool HILO = X_DT == 0;
-    constexpr int NW = kRtBlockWaves, RE = 256, TW = 16 / NW, XL = HILO ? 4 : 2;   // TW tiles of 16 experts per wave
+    constexpr int TERMS = rt_terms<X_DT>, XB = X_DT == 1 ? 2 : 4;                   // operands and bytes of an x
+    constexpr int NW = kRtBlockWaves, RE = 256, TW = 16 / NW, XL = XB;              // TW tiles of 16 experts per wave
     constexpr int SBT = RE * kRtSlab / (64 * NW);                                   // scale entries per thread and slab
-    constexpr int XS = 16 * 512;                                  // fp16 values of a slab
+    constexpr int XS = 16 * 512;                                                    // values of a slab
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int n = lane & 15, kb = lane >> 4;
     const int G = cols / 64, NS = (G + kRtSlab - 1) / kRtSlab;
     const int M0 = static_cast<int>(blockIdx.x) * 16;
 
-    __shared__ __attribute__((aligned(16))) uint16_t xs[2][HILO ? 2 : 1][XS];
+    __shared__ __attribute__((aligned(16))) uint16_t xs[2][TERMS][XS];
     __shared__ __attribute__((aligned(16))) float sbl[2][kRtSlab * (RE + 2) * 2];
     __shared__ __attribute__((aligned(16))) uint32_t wl[NW][TW][256];   // per wave: a tile's 16 rows x 64 bytes
-    __shared__ float2 xf[2][kRtSlab][16];   // (sum, 2^e) of (group, token)
+    __shared__ float xf[2][kRtSlab][16];   // sum of (group, token)
 
     // this thread's x quads and scale entries of a slab, and this wave's
     // weights of it: lane (row n, kb) bytes 16 kb .. +15 of each group
@@ -450,7 +457,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
         if (!stager) return;
         const int q = t >> 2, tok = q >> 3, g = min(kRtSlab * sl + (q & 7), G - 1);
         const char* src = static_cast<const char*>(x) +
-                          (static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 64 * g) * (HILO ? 4 : 2) + 16 * (t & 3);
+                          (static_cast<size_t>(min(M0 + tok, batch - 1)) * cols + 64 * g) * XB + 16 * (t & 3);
 #pragma unroll
         for (int i = 0; i < XL; ++i) xr[i] = *reinterpret_cast<const u32x4_t*>(src + 64 * i);
     };
@@ -479,8 +486,11 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
         }
         if (stager) {
             const int q = t >> 2, tok = q >> 3, gl = q & 7, j = t & 3;
-            const float2 xs2 = rt_stage_x<HILO>(xr, xs[buf][0], xs[buf][HILO ? 1 : 0], 512, tok, 8 * gl, j);
-            if (j == 0) xf[buf][gl][tok] = xs2;
+            uint16_t* xo[TERMS];
+#pragma unroll
+            for (int k = 0; k < TERMS; ++k) xo[k] = xs[buf][k];
+            const float sum = rt_stage_x<X_DT>(xr, xo, 512, tok, 8 * gl, j);
+            if (j == 0) xf[buf][gl][tok] = sum;
         }
     };
 
@@ -507,38 +517,19 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
         fetch_sb(nx);
 #pragma unroll
         for (int gl = 0; gl < kRtSlab; ++gl) {
-            const float2 sf = xf[buf][gl][n];
-            u32x4_t xh[2], xl[2];
+            const float sum = xf[buf][gl][n];
+            u32x4_t xv[TERMS][2];
 #pragma unroll
             for (int ks = 0; ks < 2; ++ks) {   // columns 16 kb + 8 ks .. +7 of the group
                 const int o = n * 512 + 8 * ((8 * gl + 2 * kb + ks) ^ n);
-                xh[ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][0][o]);
-                if (HILO) xl[ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][HILO ? 1 : 0][o]);
+#pragma unroll
+                for (int k = 0; k < TERMS; ++k) xv[k][ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][k][o]);
             }
 #pragma unroll
             for (int i = 0; i < TW; ++i) {
-                const u32x4_t wd = rt_tile_turn(wl[wave][i], wr[gl][i], lane);
-                u32x4_t a[2];
-#pragma unroll
-                for (int d = 0; d < 4; ++d) {
-                    uint32_t lo, hi;
-                    rt_bytes_to_f16(wd[d], lo, hi);
-                    a[d >> 1][2 * (d & 1)] = lo;
-                    a[d >> 1][2 * (d & 1) + 1] = hi;
-                }
-                f32x4_t P = f32x4_t{0.f, 0.f, 0.f, 0.f};
-                if (HILO) {
-                    P = mfma_16x16x32_f16(a[0], xl[0], P);
-                    P = mfma_16x16x32_f16(a[1], xl[1], P);
-                }
-                P = mfma_16x16x32_f16(a[0], xh[0], P);
-                P = mfma_16x16x32_f16(a[1], xh[1], P);
-                const f32x4_t* sb = reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 16 * (TW * wave + i) + 4 * kb) * 2]);
-                const f32x4_t c0 = sb[0], c1 = sb[1];
-                acc[i][0] = fmaf(c0[0], P[0] * sf.y, fmaf(c0[1], sf.x, acc[i][0]));
-                acc[i][1] = fmaf(c0[2], P[1] * sf.y, fmaf(c0[3], sf.x, acc[i][1]));
-                acc[i][2] = fmaf(c1[0], P[2] * sf.y, fmaf(c1[1], sf.x, acc[i][2]));
-                acc[i][3] = fmaf(c1[2], P[3] * sf.y, fmaf(c1[3], sf.x, acc[i][3]));
+                const f32x4_t P = rt_products<TERMS>(rt_tile_turn(wl[wave][i], wr[gl][i], lane), xv);
+                rt_accumulate(acc[i], P, sum,
+                              reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 16 * (TW * wave + i) + 4 * kb) * 2]));
             }
             fetch_w(nx, gl);
         }
@@ -599,13 +590,13 @@ hipError_t launch_router_top8(qff_ctx* ctx, hipStream_t stream, const uint32_t* 
                               float* logits, int32_t* indices, float* scores, int experts, int cols, int batch) {
     const uint16_t* s = static_cast<const uint16_t*>(scales);
     const uint16_t* b = static_cast<const uint16_t*>(biases);
-    // The kernel by the number of 16-token blocks nb (batch 8192 / 2000 / 512 /
-    // 16 at 256 x 2048, both launches, fp32 x, us):
-    //   vector units   1840 / 456 / 123 / 11.6 (bf16 x at 16: 9.5)
-    //   MFMA, 1 tile    158 / 46.4 / 17.8 / 11.2 (bf16 x at 16: 10.1)
-    //   MFMA, 2 tiles    92 / 31.8 / 14.5 / 12.4
-    //   MFMA, 4 tiles    77 / 26.4 / 17.7 / 16.6
-    //   whole blocks     58 / 28.4 / 26.4 / 26.0 (32 against 44.5 at 4096)
+    // The kernel by the number of 16-token blocks nb (batch 8192 / 4096 / 2560 /
+    // 2000 / 512 / 256 / 16 at 256 x 2048, both launches, us; fp32 x, then bf16):
+    //   vector units   1835 / 923 / 580 / 454 / 123 / 64.5 / 10.9    504 / 258 / 164 / 130 / 39.8 / 24.3 / 8.9
+    //   MFMA, 1 tile    161 / 85.3 / 57.0 / 46.4 / 17.1 / 11.8 / 11.0  103 / 55.5 / 37.9 / 31.3 / 12.8 / 10.2 / 9.5
+    //   MFMA, 2 tiles   120 / 67.1 / 46.6 / 37.9 / 14.2 / 12.9 / 12.4   65 / 36.6 / 26.4 / 22.5 / 11.4 / 11.1 / 10.7
+    //   MFMA, 4 tiles    82 / 43.9 / 35.1 / 25.2 / 17.3 / 17.3 / 17.0   58 / 33.8 / 25.6 / 20.4 / 15.4 / 15.4 / 14.8
+    //   whole blocks     64 / 33.7 / 30.4 / 30.3 / 29.1 / 28.9 / 27.7   47 / 24.6 / 23.1 / 22.8 / 23.1 / 23.0 / 21.8
     // so the tiles per workgroup grow once the grid covers the chip, and whole
     // blocks take over where they do so themselves.
     const int nb = (batch + 15) / 16, cu = ctx->num_cu;

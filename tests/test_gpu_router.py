@@ -103,6 +103,31 @@ def test_router_top8_many_tokens(hip, batch, experts, cols, xdt, sb):
     assert np.allclose(sc, p / p.sum(1, keepdims=True), atol=1e-6)
 
 
+@pytest.mark.parametrize("batch,xdt", [(2, "f32"), (17, "bf16"), (40, "f32"), (40, "bf16"), (300, "f32"),
+                                       (300, "bf16"), (1000, "f32"), (1000, "bf16"), (2600, "f32"), (2600, "bf16")])
+def test_router_logits_keep_every_bit_of_x(hip, batch, xdt):
+    """Scale 1, bias -128 and bytes of 128 except one 129 per expert: the
+    logit is one element of x. With (q - 128) x exact it is that element bit
+    for bit, also where it sits 2^-110 below the rest of its 64 columns."""
+    import qff
+    print(f"router exact x batch={batch} x={xdt}", flush=True)
+    E, C = 256, 2048
+    rng = np.random.default_rng(batch)
+    q = np.full((E, C), 128, np.uint8)
+    col = rng.permutation(C)[:E]
+    q[np.arange(E), col] = 129
+    x = (rng.uniform(1, 2, (batch, C)) * np.exp2(rng.integers(-110, 1, (batch, C)))).astype(np.float32)
+    x *= rng.choice(np.float32([-1, 1]), (batch, C))
+    if xdt == "bf16":
+        x = O.round_bf16(x)
+    xt = bf16_tensor(O.f32_to_bf16(x)) if xdt == "bf16" else f32_tensor(x)
+    one, bias = (bf16_tensor(O.f32_to_bf16(np.full((E, C // 64), v, np.float32))) for v in (1.0, -128.0))
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=1)
+    _, _, lg = qff.router_top8(ctx, torch.from_numpy(q.view(np.int32)).to(DEV), one, bias, xt)
+    torch.cuda.synchronize()
+    assert np.array_equal(lg.cpu().numpy(), x[:, col])
+
+
 def test_router_rejects_bad_calls(hip):
     import qff
     from qff._lib import lib
