@@ -51,6 +51,70 @@ namespace qff {
 template <int I>
 __device__ __forceinline__ float rt_ubyte(uint32_t v) { return static_cast<float>((v >> (8 * I)) & 0xffu); }
 
+// x[i .. i + 31] as fp32
+template <int X_DT>
+__device__ __forceinline__ void rt_load_x32(const void* x, size_t i, float (&xv)[32]) {
+    if (X_DT == 1) {
+        const uint16_t* xp = static_cast<const uint16_t*>(x) + i;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const u32x4_t u = *reinterpret_cast<const u32x4_t*>(xp + 8 * q);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                xv[8 * q + 2 * j] = __uint_as_float(u[j] << 16);
+                xv[8 * q + 2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
+            }
+        }
+    } else {
+        const float4* xp = reinterpret_cast<const float4*>(static_cast<const float*>(x) + i);
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const float4 f = xp[q];
+            xv[4 * q] = f.x;
+            xv[4 * q + 1] = f.y;
+            xv[4 * q + 2] = f.z;
+            xv[4 * q + 3] = f.w;
+        }
+    }
+}
+
+// acc + scale * sum(q x) + bias * sum(x) of half a group: 32 weight bytes and x
+__device__ __forceinline__ float rt_half_group(const u32x4_t (&wq)[2], const float (&xv)[32], float scale, float bias,
+                                               float acc) {
+    float dot = 0.0f, sum = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const uint32_t wd = wq[j >> 2][j & 3];
+        dot = fmaf(rt_ubyte<0>(wd), xv[4 * j], dot);
+        dot = fmaf(rt_ubyte<1>(wd), xv[4 * j + 1], dot);
+        dot = fmaf(rt_ubyte<2>(wd), xv[4 * j + 2], dot);
+        dot = fmaf(rt_ubyte<3>(wd), xv[4 * j + 3], dot);
+        sum += (xv[4 * j] + xv[4 * j + 1]) + (xv[4 * j + 2] + xv[4 * j + 3]);
+    }
+    acc = fmaf(scale, dot, acc);
+    return fmaf(bias, sum, acc);
+}
+
+// One logit by one wave, in the operations and order of router_logits_kernel.
+template <int SB_DT, int X_DT>
+__device__ __forceinline__ float rt_vector_logit(const uint32_t* w, const uint16_t* scales, const uint16_t* biases,
+                                                 const void* x, int cols, int m, int e, int lane) {
+    const int G = cols / 64, npc = cols / 32;
+    float acc = 0.0f;
+    for (int p0 = 0; p0 < npc; p0 += 64) {
+        const int pc = min(p0 + lane, npc - 1);
+        const bool live = p0 + lane < npc;
+        const u32x4_t* src = reinterpret_cast<const u32x4_t*>(w + static_cast<size_t>(e) * (cols / 4) + 8 * pc);
+        const u32x4_t wq[2] = {src[0], src[1]};
+        const size_t gi = static_cast<size_t>(e) * G + pc / 2;
+        float xv[32];
+        rt_load_x32<X_DT>(x, static_cast<size_t>(m) * cols + 32 * pc, xv);
+        acc = rt_half_group(wq, xv, live ? elem<SB_DT>::load(scales, gi) : 0.0f,
+                            live ? elem<SB_DT>::load(biases, gi) : 0.0f, acc);
+    }
+    return group_sum<64>(acc);
+}
+
 // grid (ceil(E / 4), ceil(batch / NT)), 256 threads; KW = 2048-column pieces
 template <int SB_DT, int X_DT, int KW, int NT>
 __global__ __launch_bounds__(256) void router_logits_kernel(const uint32_t* __restrict__ w,
@@ -88,43 +152,9 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const uint32_t* __re
         for (int k = 0; k < KW; ++k) {
             const int pcc = min(lane + 64 * k, npc - 1);
             float xv[32];
-            if (X_DT == 1) {
-                const uint16_t* xp = static_cast<const uint16_t*>(x) + static_cast<size_t>(m) * cols + 32 * pcc;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const u32x4_t u = *reinterpret_cast<const u32x4_t*>(xp + 8 * q);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        xv[8 * q + 2 * j] = __uint_as_float(u[j] << 16);
-                        xv[8 * q + 2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
-                    }
-                }
-            } else {
-                const float4* xp =
-                    reinterpret_cast<const float4*>(static_cast<const float*>(x) + static_cast<size_t>(m) * cols + 32 * pcc);
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    const float4 f = xp[q];
-                    xv[4 * q] = f.x;
-                    xv[4 * q + 1] = f.y;
-                    xv[4 * q + 2] = f.z;
-                    xv[4 * q + 3] = f.w;
-                }
-            }
-            float dot = 0.0f, sum = 0.0f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const uint32_t wd = wq[k][j >> 2][j & 3];
-                dot = fmaf(rt_ubyte<0>(wd), xv[4 * j], dot);
-                dot = fmaf(rt_ubyte<1>(wd), xv[4 * j + 1], dot);
-                dot = fmaf(rt_ubyte<2>(wd), xv[4 * j + 2], dot);
-                dot = fmaf(rt_ubyte<3>(wd), xv[4 * j + 3], dot);
-                sum += (xv[4 * j] + xv[4 * j + 1]) + (xv[4 * j + 2] + xv[4 * j + 3]);
-            }
+            rt_load_x32<X_DT>(x, static_cast<size_t>(m) * cols + 32 * pcc, xv);
             // half a group per lane; pieces past the row end (cols < 2048) add nothing
-            const float sk = live[k] ? sv[k] : 0.0f, bk = live[k] ? bv[k] : 0.0f;
-            acc = fmaf(sk, dot, acc);
-            acc = fmaf(bk, sum, acc);
+            acc = rt_half_group(wq[k], xv, live[k] ? sv[k] : 0.0f, live[k] ? bv[k] : 0.0f, acc);
         }
         accs[mi] = group_sum<64>(acc);
     }
@@ -150,25 +180,33 @@ __device__ __forceinline__ void rt_bytes_to_bf16(uint32_t w, uint32_t& lo, uint3
     hi = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
 }
 
+// Tokens with an infinity or values near fp32's largest have their logits from
+// rt_vector_logit: an infinity leaves no terms (inf - inf), and q - 128 can
+// pass fp32's range where q, with the other sign or zero, does not.
+constexpr float kRtRange = 0x1p96f;
+
 // One group (64 columns) of one token, held by the four lanes j of a quad (fp32:
 // columns 16 i + 4 j .. +3 in piece i; bf16: 32 i + 8 j .. +7), as bf16
 // operands: a bf16 x as it is, an fp32 x as the three terms that cutting 8
 // significant bits off at a time leaves, hi + mid + lo == x with every bit (of
 // |x| >= 2^-110: below that the last term meets bf16's smallest step, 2^-133).
 // Term k goes to xo[k], LDS rows [token][row] at 16-byte pieces p0 + c,
-// swizzled by the token. Returns the sum of x.
+// swizzled by the token. Returns the sum of x; redo becomes true where the
+// lane has an |x| of kRtRange or more (a NaN makes every logit NaN either way).
 template <int X_DT, int XL>
 __device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* const (&xo)[rt_terms<X_DT>], int row,
-                                            int tok, int p0, int j) {
+                                            int tok, int p0, int j, bool& redo) {
     const int sw = tok & (row / 8 - 1) & 15;
-    float sum = 0.0f;
+    float sum = 0.0f, mx = 0.0f;
     if constexpr (X_DT == 1) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                sum += __uint_as_float(xr[i][c] << 16);
-                sum += __uint_as_float(xr[i][c] & 0xffff0000u);
+                const float v0 = __uint_as_float(xr[i][c] << 16), v1 = __uint_as_float(xr[i][c] & 0xffff0000u);
+                sum += v0;
+                sum += v1;
+                mx = fmaxf(fmaxf(mx, fabsf(v0)), fabsf(v1));
             }
             *reinterpret_cast<u32x4_t*>(xo[0] + tok * row + 8 * ((p0 + 4 * i + j) ^ sw)) = xr[i];
         }
@@ -180,6 +218,7 @@ __device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* c
             for (int c = 0; c < 4; ++c) {
                 const float v = __uint_as_float(xr[i][c]);
                 sum += v;
+                mx = fmaxf(mx, fabsf(v));
                 f[0][c] = xr[i][c];
                 const float r1 = v - __uint_as_float(f[0][c] & 0xffff0000u);
                 f[1][c] = __float_as_uint(r1);
@@ -192,6 +231,7 @@ __device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* c
                                                                  __builtin_amdgcn_perm(f[k][3], f[k][2], 0x07060302u)};
         }
     }
+    redo |= mx >= kRtRange;
     return group_sum<4>(sum);
 }
 
@@ -260,6 +300,9 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
     __shared__ __attribute__((aligned(16))) uint32_t wl[NW][256];
     __shared__ __attribute__((aligned(16))) uint16_t xl[NW][TERMS][16 * 64];
     __shared__ float xf[NW][16];
+    __shared__ unsigned redo_s;   // bit per token: redone on the vector units
+    bool redo = false;
+    if (t == 0) redo_s = 0;
 
     const char* xrow = static_cast<const char*>(x) +
                        static_cast<size_t>(min(M0 + (lane >> 2), batch - 1)) * cols * XB + 16 * (lane & 3);
@@ -304,7 +347,7 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
         uint16_t* xo[TERMS];
 #pragma unroll
         for (int k = 0; k < TERMS; ++k) xo[k] = xl[wave][k];
-        const float xs = rt_stage_x<X_DT>(xr[s], xo, 64, lane >> 2, 0, lane & 3);
+        const float xs = rt_stage_x<X_DT>(xr[s], xo, 64, lane >> 2, 0, lane & 3, redo);
         if ((lane & 3) == 0) xf[wave][lane >> 2] = xs;
         __builtin_amdgcn_wave_barrier();
         const float sum = xf[wave][n];
@@ -329,16 +372,26 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
         if (g + NW < G) step(1, g + NW);
         if (g + 3 * NW < G) fetch(1, g + 3 * NW);
     }
+    if (redo) atomicOr(&redo_s, 1u << (lane >> 2));
     __syncthreads();   // the scales are consumed; their bytes take the partial sums
 #pragma unroll
     for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4_t*>(&lds[wave * RE * 16 + (i * 64 + lane) * 4]) = acc[i];
     __syncthreads();
+    const unsigned rd = redo_s;
     for (int o = t; o < RE * 16; o += 64 * NW) {
         float v = lds[o];
 #pragma unroll
         for (int ww = 1; ww < NW; ++ww) v += lds[ww * RE * 16 + o];
         const int l = (o >> 2) & 63, e = E0 + 16 * (o >> 8) + 4 * (l >> 4) + (o & 3), m = M0 + (l & 15);
-        if (m < batch && e < experts) logits[static_cast<size_t>(m) * experts + e] = v;
+        if (m < batch && e < experts && !(rd >> (l & 15) & 1)) logits[static_cast<size_t>(m) * experts + e] = v;
+    }
+    if (rd == 0) return;   // workgroup-uniform
+    for (int tok = 0; tok < min(16, batch - M0); ++tok) {
+        if (!(rd >> tok & 1)) continue;
+        for (int e = E0 + wave; e < min(E0 + RE, experts); e += NW) {
+            const float v = rt_vector_logit<SB_DT, X_DT>(w, scales, biases, x, cols, M0 + tok, e, lane);
+            if (lane == 0) logits[static_cast<size_t>(M0 + tok) * experts + e] = v;
+        }
     }
 }
 
@@ -442,6 +495,9 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     __shared__ __attribute__((aligned(16))) float sbl[2][kRtSlab * (RE + 2) * 2];
     __shared__ __attribute__((aligned(16))) uint32_t wl[NW][TW][256];   // per wave: a tile's 16 rows x 64 bytes
     __shared__ float xf[2][kRtSlab][16];   // sum of (group, token)
+    __shared__ unsigned redo_s;   // bit per token: redone on the vector units
+    bool redo = false;
+    if (t == 0) redo_s = 0;
 
     // this thread's x quads and scale entries of a slab, and this wave's
     // weights of it: lane (row n, kb) bytes 16 kb .. +15 of each group
@@ -489,7 +545,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
             uint16_t* xo[TERMS];
 #pragma unroll
             for (int k = 0; k < TERMS; ++k) xo[k] = xs[buf][k];
-            const float sum = rt_stage_x<X_DT>(xr, xo, 512, tok, 8 * gl, j);
+            const float sum = rt_stage_x<X_DT>(xr, xo, 512, tok, 8 * gl, j, redo);
             if (j == 0) xf[buf][gl][tok] = sum;
         }
     };
@@ -540,12 +596,23 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     // lane: token n, experts 32 wave + 16 i + 4 kb .. +3
     // every expert of the 16 tokens is here: logits through LDS (the staging
     // buffers are idle once every wave is past its last slab)
+    if (redo) atomicOr(&redo_s, 1u << (t >> 5));   // the token of quad t / 4
     __syncthreads();
     float* lg = reinterpret_cast<float*>(xs);   // [16][RE + 4]
 #pragma unroll
     for (int i = 0; i < TW; ++i)
         *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 16 * (TW * wave + i) + 4 * kb]) = tot[i];
     __syncthreads();
+    if (const unsigned rd = redo_s; rd != 0) {   // workgroup-uniform
+        for (int tok = 0; tok < min(16, batch - M0); ++tok) {
+            if (!(rd >> tok & 1)) continue;
+            for (int e = wave; e < experts; e += NW) {
+                const float v = rt_vector_logit<SB_DT, X_DT>(w, scales, biases, x, cols, M0 + tok, e, lane);
+                if (lane == 0) lg[tok * (RE + 4) + e] = v;
+            }
+        }
+        __syncthreads();
+    }
     for (int tok = wave; tok < 16; tok += NW) {
         const int m = M0 + tok;
         if (m >= batch) break;

@@ -128,6 +128,45 @@ def test_router_logits_keep_every_bit_of_x(hip, batch, xdt):
     assert np.array_equal(lg.cpu().numpy(), x[:, col])
 
 
+@pytest.mark.parametrize("batch,experts,cols,xdt,sb", [(4, 256, 2048, "f32", "bf16"), (40, 256, 4096, "bf16", "f16"),
+                                                       (300, 250, 2048, "bf16", "bf16"), (300, 256, 64, "f32", "f16"),
+                                                       (1000, 256, 2048, "f32", "bf16"), (1000, 40, 320, "bf16", "f16"),
+                                                       (2600, 256, 2048, "f32", "f16"), (2600, 100, 576, "bf16", "bf16")])
+def test_router_special_tokens(hip, batch, experts, cols, xdt, sb):
+    """Tokens with infinities, NaN or magnitudes up to 2^127 in a batch: their
+    logits and ranking are bit for bit those of a call with that token alone,
+    and the other tokens' those of a batch that has zeros in their place."""
+    import qff
+    print(f"router special tokens batch={batch} experts={experts} cols={cols} x={xdt} scales={sb}", flush=True)
+    w, s, b = synth.q8_weight(experts, cols, seed=experts + cols + batch, sb_dtype=sb)
+    rng = np.random.default_rng(batch + cols)
+    conv = f16_tensor if sb == "f16" else bf16_tensor
+    # biases of both signs: q x and b sum(x) both infinite, of one sign or two
+    bf = rng.choice(np.float32([-0.2, 0.05]), b.shape)
+    wt = (torch.from_numpy(w.view(np.int32)).to(DEV), conv(s), conv(O.f32_to_f16(bf) if sb == "f16" else O.f32_to_bf16(bf)))
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    spec = sorted({0, 1, batch // 2, batch - 1} if batch > 4 else {0, 1, 2})
+    plain = x.copy()
+    plain[spec] = 0.0
+    x[spec[0], 5] = np.inf
+    x[spec[1], [3, cols - 1]] = np.inf, -np.inf
+    x[spec[2]] *= 2.0 ** 124
+    if len(spec) > 3:
+        x[spec[3], cols // 2] = np.nan
+    mk = (lambda v: bf16_tensor(O.f32_to_bf16(v))) if xdt == "bf16" else f32_tensor
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=1)
+    xt = mk(x)
+    idx, sc, lg = (t.cpu().numpy() for t in qff.router_top8(ctx, *wt, xt))
+    pidx, _, plg = (t.cpu().numpy() for t in qff.router_top8(ctx, *wt, mk(plain)))
+    rest = np.setdiff1d(np.arange(batch), spec)
+    assert np.array_equal(lg[rest], plg[rest]) and np.array_equal(idx[rest], pidx[rest])
+    for m in spec:
+        i1, s1, l1 = (t.cpu().numpy()[0] for t in qff.router_top8(ctx, *wt, xt[m:m + 1].clone()))
+        assert np.array_equal(lg[m], l1, equal_nan=True), m
+        assert np.array_equal(idx[m], i1) and np.array_equal(sc[m], s1, equal_nan=True)
+    assert np.isinf(lg[spec[0]]).any()   # where the bias is positive
+
+
 def test_router_rejects_bad_calls(hip):
     import qff
     from qff._lib import lib
