@@ -1482,9 +1482,9 @@ static Q4Parts q4_pack_parts(const qff_q4_part* parts, int nparts, int rpb, int&
     return P;
 }
 
-// Many tokens: x16 and the per-token factors once per token slice, then one
-// tiled launch over all parts (the small parts' tiles fill the chip beside the
-// large one's).
+// Many tokens: per token slice x16 and the per-token factors, then one tiled
+// launch over the parts (the small parts' tiles fill the chip beside the large
+// one's); twice where the parts need both kernels, whose x16 orders differ.
 template <bool NORM>
 static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_part* parts, int nparts,
                                 qff_dtype sb_dtype, const void* x, qff_dtype x_dtype, const Q4Norm& norm,
@@ -1493,10 +1493,10 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
     const int lds = G * kQ4GemmRows * 4;   // packed (s, b) of the row tile
     QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<1>>(lds)));
     QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<2>>(lds)));
-    // Which kernel: by the tokens and columns alone, and K always split in
-    // four, so that a part's sums do not depend on the rows beside it
-    // (scales and biases are read two groups at a time: an even number of
-    // groups, 4-byte-aligned scale rows). Which tile: the largest that
+    // Which kernel: part by part, and K always split in four, so that a part's
+    // sums do not depend on the rows beside it (the split tiles read scales
+    // and biases two groups at a time: an even number of groups,
+    // 4-byte-aligned scale rows). Which split tile: the largest that
     // still covers the chip. fp32 x, x16 pass included, us at 64 / 200 /
     // 448 / 512 / 1000 / 4096 tokens:
     //   2048 x 4096, 256 x 128 tiles    73 / 97 / - / 99 / 99 / 149
@@ -1511,62 +1511,70 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
     // The widest in-projection sets the line at 2048 columns. The large tile
     // stages the scales of all of K in LDS and so runs one workgroup a CU
     // above that: it takes over later there.
-    bool split = (cols / 64) % 2 == 0 && batch <= (cols > 2048 ? 4096 : 448);
-    for (int i = 0; i < nparts; ++i)
-        split = split && ((reinterpret_cast<uintptr_t>(parts[i].scales) | reinterpret_cast<uintptr_t>(parts[i].biases)) & 3) == 0;
+    const auto takes_split = [&](const qff_q4_part& q) {
+        return (cols / 64) % 2 == 0 && batch <= (cols > 2048 ? 4096 : 448) &&
+               ((reinterpret_cast<uintptr_t>(q.scales) | reinterpret_cast<uintptr_t>(q.biases)) & 3) == 0;
+    };
+    const int cu = ctx->num_cu, pm = (1 << 20) / std::max(G / 2, 1) + 1;   // idx / (G / 2) = idx pm >> 20, idx < 2048
     for (int m0 = 0; m0 < batch; m0 += ctx->q4_xs_tokens) {
         const int mb = min(ctx->q4_xs_tokens, batch - m0);
         const void* xm = static_cast<const char*>(x) + static_cast<size_t>(m0) * cols * (x_dtype == QFF_BF16 ? 2 : 4);
-        {
-            ProfScope prof(ctx, stream, "q4_x16");
-            // four waves a token below 768 tokens (2048 x 4096 product, both
-            // launches: 11.3 against 12.3 us at 33, 16.4 / 17.3 at 200; equal at
-            // 768, 140 / 131 at 4096)
+        for (const bool split : {true, false}) {
+            // the class's parts, outputs offset to this slice
+            qff_q4_part sl[QFF_Q4_MAX_PARTS];
+            int n = 0;
+            for (int i = 0; i < nparts; ++i) {
+                if (takes_split(parts[i]) != split) continue;
+                sl[n] = parts[i];
+                const size_t yoff = static_cast<size_t>(m0) * parts[i].rows * (parts[i].y_dtype == QFF_BF16 ? 2 : 4);
+                sl[n].y = static_cast<char*>(parts[i].y) + yoff;
+                if (parts[i].residual) sl[n].residual = static_cast<const char*>(parts[i].residual) + yoff;
+                ++n;
+            }
+            if (n == 0) continue;
+            {
+                ProfScope prof(ctx, stream, "q4_x16");
+                // four waves a token below 768 tokens (2048 x 4096 product, both
+                // launches: 11.3 against 12.3 us at 33, 16.4 / 17.3 at 200; equal at
+                // 768, 140 / 131 at 4096)
 #define QFF_X16(X)                                                                                                       \
     if (!split) q4_x16_kernel<X, NORM, 1, 4, true><<<(mb + 3) / 4, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);     \
     else if (mb < 768) q4_x16_kernel<X, NORM, 4, 1, false><<<mb, 256, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm);      \
     else q4_x16_kernel<X, NORM, 1, 8, false><<<(mb + 7) / 8, 512, 0, stream>>>(xm, ctx->q4_x16, ctx->q4_fm, cols, mb, norm)
-            if (x_dtype == QFF_BF16) { QFF_X16(1); } else { QFF_X16(0); }
+                if (x_dtype == QFF_BF16) { QFF_X16(1); } else { QFF_X16(0); }
 #undef QFF_X16
-        }
-        // one launch over every part's row tiles, outputs offset to this slice
-        qff_q4_part sl[QFF_Q4_MAX_PARTS];
-        for (int i = 0; i < nparts; ++i) {
-            sl[i] = parts[i];
-            const size_t yoff = static_cast<size_t>(m0) * parts[i].rows * (parts[i].y_dtype == QFF_BF16 ? 2 : 4);
-            sl[i].y = static_cast<char*>(parts[i].y) + yoff;
-            if (parts[i].residual) sl[i].residual = static_cast<const char*>(parts[i].residual) + yoff;
-        }
-        const auto pack_grid = [&](int rpb, int tpb, Q4Parts& P) {
-            int tiles = 0;
-            P = q4_pack_parts(sl, nparts, rpb, tiles);
-            return dim3(tiles, (mb + tpb - 1) / tpb);
-        };
-        const auto count = [](dim3 g) { return static_cast<int>(g.x * g.y); };
-        Q4Parts P;
-        ProfScope prof(ctx, stream, "q4_gemm");
-        const int cu = ctx->num_cu, pm = (1 << 20) / std::max(G / 2, 1) + 1;   // idx / (G / 2) = idx pm >> 20, idx < 2048
-        dim3 grid;
+            }
+            // one launch over the parts' row tiles
+            const auto pack_grid = [&](int rpb, int tpb, Q4Parts& P) {
+                int tiles = 0;
+                P = q4_pack_parts(sl, n, rpb, tiles);
+                return dim3(tiles, (mb + tpb - 1) / tpb);
+            };
+            const auto count = [](dim3 g) { return static_cast<int>(g.x * g.y); };
+            Q4Parts P;
+            ProfScope prof(ctx, stream, "q4_gemm");
+            dim3 grid;
 #define QFF_SPLIT(RT, MT, WK, D)                                                                               \
     if (sb_dtype == QFF_BF16)                                                                                  \
         q4_gemm_split_kernel<1, RT, MT, WK, D><<<grid, 64 * WK, 0, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb, pm); \
     else                                                                                                       \
         q4_gemm_split_kernel<2, RT, MT, WK, D><<<grid, 64 * WK, 0, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb, pm)
-        if (!split) {
-            grid = pack_grid(kQ4GemmRows, kQ4GemmToks, P);
-            if (sb_dtype == QFF_BF16)
-                q4_gemm_kernel<1><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
-            else
-                q4_gemm_kernel<2><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
-        } else if (count(grid = pack_grid(32, 32, P)) <= cu) {
-            QFF_SPLIT(1, 1, 4, 2);
-        } else if (count(grid = pack_grid(32, 64, P)) <= cu) {
-            QFF_SPLIT(1, 2, 4, 1);
-        } else {
-            grid = pack_grid(64, 64, P);
-            QFF_SPLIT(2, 2, 4, 1);
-        }
+            if (!split) {
+                grid = pack_grid(kQ4GemmRows, kQ4GemmToks, P);
+                if (sb_dtype == QFF_BF16)
+                    q4_gemm_kernel<1><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
+                else
+                    q4_gemm_kernel<2><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
+            } else if (count(grid = pack_grid(32, 32, P)) <= cu) {
+                QFF_SPLIT(1, 1, 4, 2);
+            } else if (count(grid = pack_grid(32, 64, P)) <= cu) {
+                QFF_SPLIT(1, 2, 4, 1);
+            } else {
+                grid = pack_grid(64, 64, P);
+                QFF_SPLIT(2, 2, 4, 1);
+            }
 #undef QFF_SPLIT
+        }
     }
     return hipGetLastError();
 }

@@ -364,6 +364,28 @@ def test_q4_many_tokens_split_tiles(hip, batch, cols, odd):
         assert _rel(got, ref) <= (1e-3 if dt == torch.float32 else 4e-3)
 
 
+@pytest.mark.parametrize("batch,cols", [(40, 4096), (70, 2048), (300, 2048)])
+def test_q4_part_does_not_depend_on_the_parts_beside_it(hip, batch, cols):
+    """A part's outputs bit for bit the same alone and beside others: one with
+    scale rows at odd addresses (the other kernel), one of many rows (other
+    tiles)."""
+    import qff
+    print(f"q4 parts beside others batch={batch} cols={cols}", flush=True)
+    ws = [_w_gpu(*synth.q4_weight(r, cols, seed=r, sb_dtype="bf16"), "bf16") for r in (100, 256, 8192)]
+    w, s, b = ws[1]
+    ws[1] = (w, *(torch.cat([v.new_zeros(1), v.flatten()])[1:].view(v.shape) for v in (s, b)))
+    rng = np.random.default_rng(batch)
+    x, nw = f32_tensor(rng.standard_normal((batch, cols))), f32_tensor(1 + 0.1 * rng.standard_normal(cols))
+    res = [f32_tensor(rng.standard_normal((batch, t[0].shape[0]))) for t in ws]
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=64)
+    both = qff.q4_norm_matmul_parts(ctx, ws, x, nw, 1e-6, residuals=res)
+    torch.cuda.synchronize()
+    for i, t in enumerate(ws):
+        alone, = qff.q4_norm_matmul_parts(ctx, [t], x, nw, 1e-6, residuals=[res[i]])
+        torch.cuda.synchronize()
+        assert torch.equal(alone, both[i]), i
+
+
 def test_q4_norm_matmul_parts_rejects_bad_calls(hip):
     import qff
     from qff._lib import Q4Part, lib
