@@ -386,6 +386,30 @@ def test_q4_part_does_not_depend_on_the_parts_beside_it(hip, batch, cols):
         assert torch.equal(alone, both[i]), i
 
 
+@pytest.mark.parametrize("rows,cols,batch,over", [(32768, 2048, 200, 449), (32768 + 5, 2048, 130, 449),
+                                                  (8192, 3072, 1100, 4097), (32768, 4096, 512, 4097)])
+def test_q4_wide_part_takes_the_large_tile(hip, rows, cols, batch, over):
+    """A part whose own large tiles fill the chip: its outputs are bit for bit
+    those of the first tokens of a batch that always takes that tile, within
+    1e-3 of the fp64 product (256 sampled rows), a narrow part beside it too."""
+    import qff
+    print(f"q4 wide part {rows}x{cols} batch={batch}", flush=True)
+    ws = [synth.q4_weight(r, cols, seed=r + batch, sb_dtype="bf16") for r in (rows, 100)]
+    x = torch.empty(over, cols, device=DEV).normal_(generator=torch.Generator(device=DEV).manual_seed(batch))
+    gw = [_w_gpu(*w, "bf16") for w in ws]
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=4096)
+    big, = qff.q4_matmul_parts(ctx, gw[:1], x)
+    big = big[:batch].clone()
+    wide, narrow = qff.q4_matmul_parts(ctx, gw, x[:batch])
+    torch.cuda.synchronize()
+    assert torch.equal(wide, big)
+    x64 = x[:batch].double().cpu().numpy()
+    pick = np.unique(np.r_[0, rows - 1, np.random.default_rng(rows).integers(0, rows, 254)])
+    for (w, s, b), out, sel in ((ws[0], wide, pick), (ws[1], narrow, np.arange(100))):
+        ref = x64 @ O.q4_dequant(w[sel], s[sel], b[sel], O.BF16).astype(np.float64).T
+        assert _rel(out[:, torch.from_numpy(sel).to(DEV)].double().cpu().numpy(), ref) <= 1e-3
+
+
 def test_q4_norm_matmul_parts_rejects_bad_calls(hip):
     import qff
     from qff._lib import Q4Part, lib
