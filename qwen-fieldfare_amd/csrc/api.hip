@@ -26,10 +26,15 @@ static qff_ctx_cfg resolve(const qff_ctx_cfg* cfg) {
 // Tokens per slice of a many-token Q4 product (fp16 activations in workspace).
 int q4_xs_tokens(const qff_ctx_cfg& cfg) { return std::max(std::max(cfg.max_batch, cfg.max_prefill_tokens), 1024); }
 
-int pf_slots(const qff_ctx_cfg& cfg) {
-    const long long tc = (static_cast<long long>(cfg.max_prefill_tokens) + 63) / 64 * 64;
-    const long long tiles = (static_cast<long long>(cfg.max_ctx) + 63) / 64;
-    return static_cast<int>(std::max(tc, std::min(3072ll, tc * std::max(1ll, tiles / 4))));
+long long pf_slots(const qff_ctx_cfg& cfg) {
+    const int tokens = cfg.max_prefill_tokens, tiles = cfg.max_ctx / 64 + (cfg.max_ctx % 64 != 0);
+    constexpr int kCus = 256;   // of gfx950: as many shares as a call can have
+    long long slots = (tokens + 63ll) / 64 * 64;
+    for (int blocks = 1; blocks <= kCus / 2; ++blocks) {
+        const int t = std::min(16 * blocks, tokens);
+        slots = std::max(slots, 1ll * t * pf_shares(kCus, t, tiles));
+    }
+    return slots;
 }
 
 WorkspaceLayout workspace_layout(const qff_ctx_cfg& cfg) {

@@ -730,16 +730,15 @@ hipError_t launch_gqa_prefill(qff_ctx* ctx, hipStream_t stream, const qff_gqa_pa
     }
     const int vt_stride = (ctx->cfg.max_ctx + kPfKT - 1) / kPfKT;
     const int nqb = (T + kPfQB - 1) / kPfQB, ntiles = (start_pos + T + kPfKT - 1) / kPfKT;
-    // Shares of the tiles per block: enough to give every CU one workgroup, of
-    // four tiles or more each, no more than the first block has tiles (none is
-    // empty; a prompt from position 0 is not shared) nor than the partial
-    // slots. us per call, one share / this rule / the best of 1 .. 64:
+    // Shares of the tiles per block: pf_shares, no more than the first block has
+    // tiles (none is empty; a prompt from position 0 is not shared) nor than the
+    // partial slots. us per call, one share / this rule / the best of 1 .. 64:
     //   16 tokens at 2000, 12000, 60000   64 / 31 / 30, 253 / 39 / 39, 1477 / 82 / 82
     //   128 at 2000, 12000                69 / 37 / 37, 257 / 61 / 60
     //   500 at 3000, 12011                97 / 59 / 59, 265 / 129 / 129
     //   1000 at 2000, 8000                88 / 76 / 76, 201 / 168 / 168
-    int shares = std::min(std::min(ctx->num_cu / (2 * nqb), ntiles / 4), std::min(64, start_pos / kPfKT + 1));
-    shares = std::max(1, std::min(shares, ctx->pf_slots / T));
+    int shares = std::min(pf_shares(ctx->num_cu, T, ntiles), start_pos / kPfKT + 1);
+    shares = static_cast<int>(std::max(1ll, std::min<long long>(shares, ctx->pf_slots / T)));
     float2* md = reinterpret_cast<float2*>(ctx->pf_md);
     {
         ProfScope prof(ctx, stream, "gqa_prefill_attn");

@@ -56,7 +56,7 @@ struct qff_ctx {
     // bytes, and their (m, d) pairs.
     float* pf_o = nullptr;
     float* pf_md = nullptr;   // [pf_slots][16][2]
-    int pf_slots = 0;
+    long long pf_slots = 0;
     qff_dn_bufs dn{};
     // DeltaNet decode: per (sequence, key head) arrival counters [max_batch][16],
     // zero between launches (the second arrival resets its counter).
@@ -78,10 +78,18 @@ constexpr int kGqaSeqChunks = 128;     // partial slots per (sequence, kv head) 
 // (sequence, kv head, chunk) partial slots of the workspace: a call with a
 // smaller batch spreads them over more chunks per sequence.
 inline int gqa_slots(const qff_ctx_cfg& cfg) { return 2 * (cfg.max_batch > 4 ? cfg.max_batch : 4) * kGqaSeqChunks; }
-// (share, token) slots of a full-attention prefill in shares: as many as its
-// longest call can use, 3072 (a share of every CU and half as many again) at
-// most where that exceeds a call's tokens.
-int pf_slots(const qff_ctx_cfg& cfg);
+// Shares of each 16-token block's 64-position tiles in a full-attention
+// prefill: enough to give every CU one workgroup (two kv heads), of four tiles
+// or more each, 64 at most.
+inline int pf_shares(int cus, int tokens, int tiles) {
+    const int per_cu = cus / (2 * ((tokens + 15) / 16)), by_tiles = tiles / 4;
+    const int s = per_cu < by_tiles ? per_cu : by_tiles;
+    return s < 1 ? 1 : s > 64 ? 64 : s;
+}
+// (share, token) slots of the workspace: as many as any call the configuration
+// allows can use (none beyond its tokens for a context of one-token prefills,
+// 2048 from 33 tokens on), and the DeltaNet prefill's tokens in whole chunks.
+long long pf_slots(const qff_ctx_cfg& cfg);
 constexpr int kSchedSlots = 8;         // work-queue counter pairs in the context
 constexpr int kQ4SkSlots = 4096;       // (row tile, slice) partials of the split decode-batch Q4 product
 constexpr int kSchedChunkLocal = 0;    // slot of the DeltaNet chunk-local pass

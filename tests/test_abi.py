@@ -73,6 +73,26 @@ def test_workspace_size_and_argument_checks_without_gpu():
     assert L.qff_router_top8(N, N, N, N, N, 1, N, 0, N, N, N, 256, 2048, 1) == -1
 
 
+def test_workspace_grows_with_the_context_by_what_its_calls_use():
+    """From 64 to 65536 positions the workspace gains the fp16 K and transposed
+    V copies (1 KB a position each) and the partial rows of a prefill whose
+    tiles are shared out (16512 bytes a slot): 64 shares of up to 16 tokens,
+    2048 slots at most, none for a context of one-token prefills, whose 64
+    slots the DeltaNet chunk already needs."""
+    import qff
+    from qff._lib import CtxCfg
+    L = qff.lib()
+    size = {}
+    for P in (1, 2, 16, 17, 64, 300, 2048, 8192):
+        for C in (64, 65536):
+            n = ctypes.c_size_t()
+            assert L.qff_workspace_size(ctypes.byref(CtxCfg(4, C, P)), ctypes.byref(n)) == 0
+            size[C] = n.value
+        slots = max([min(16 * k, P) * min(64, 128 // k) for k in range(1, 129)])
+        extra = max(0, slots - (P + 63) // 64 * 64) * (4096 + 32) * 4
+        assert size[65536] - size[64] == 2 * (65536 - 64) * 1024 + extra, P
+
+
 def test_product_has_no_cpu_fallback():
     """The product package never imports the oracle."""
     pkg = os.path.join(ROOT, "qwen-fieldfare_amd")
