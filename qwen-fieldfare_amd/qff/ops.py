@@ -235,10 +235,16 @@ def router_top8(ctx: Context, w, scales, biases, x: torch.Tensor, logits=None, i
     return indices, scores, logits
 
 
+def _require_f32(**tensors):
+    for name, t in tensors.items():
+        if t.dtype != _f32:
+            raise TypeError(f"{name} must be float32")
+
+
 def _dn_params(p: dict, eps: float) -> bytes:
     a_log, dt_bias, conv_w, norm_w = p["a_log"], p["dt_bias"], p["conv_w"], p["norm_w"]
     if a_log.dtype != _f32 or dt_bias.dtype != _f32 or conv_w.dtype != _f32 or norm_w.dtype != _f32:
-        raise TypeError("a_log, dt_bias, conv_w and norm_w must be float32")
+        _require_f32(a_log=a_log, dt_bias=dt_bias, conv_w=conv_w, norm_w=norm_w)
     return _pack(_P_DN, (_ptr(a_log), _ptr(dt_bias), _ptr(conv_w), _ptr(norm_w)), eps)
 
 
@@ -248,7 +254,7 @@ def _check_dn_inputs(qkv, z, a, b, conv_state, ssm_state, n, seqs):
     if z.dtype != qkv.dtype:
         raise TypeError("qkv and z must share a dtype")
     if a.dtype != _f32 or b.dtype != _f32 or conv_state.dtype != _f32 or ssm_state.dtype != _f32:
-        raise TypeError("a, b, conv_state and ssm_state must be float32")
+        _require_f32(a=a, b=b, conv_state=conv_state, ssm_state=ssm_state)
     if qkv.numel() != n * 8192 or z.numel() != n * 4096 or a.numel() != n * 32 or b.numel() != n * 32:
         raise ValueError("qkv, z, a, b must be [n, 8192], [n, 4096], [n, 32], [n, 32]")
     if conv_state.numel() != seqs * 8192 * 4 or ssm_state.numel() != seqs * 32 * 128 * 128:

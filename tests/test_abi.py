@@ -136,6 +136,21 @@ def test_parameter_structs_match_the_header(tmp_path):
             assert int(got[f"{cname} {fname}"]) == getattr(py, fname).offset, (cname, fname)
 
 
+def test_wrong_dtypes_are_reported_by_name():
+    import torch
+    from qff import ops
+    names = ("a_log", "dt_bias", "conv_w", "norm_w")
+    for bad in names:
+        p = {k: torch.zeros(4, dtype=torch.float64 if k == bad else torch.float32) for k in names}
+        with pytest.raises(TypeError, match=f"^{bad} must be float32$"):
+            ops._dn_params(p, 1e-6)
+    names = ("a", "b", "conv_state", "ssm_state")
+    for bad in names:
+        t = [torch.zeros(4, dtype=torch.bfloat16 if k == bad else torch.float32) for k in names]
+        with pytest.raises(TypeError, match=f"^{bad} must be float32$"):
+            ops._check_dn_inputs(torch.zeros(4), torch.zeros(4), *t, 1, 1)
+
+
 def test_packed_parameter_blocks_match_the_structures():
     """The bytes ops.py hands over are the ctypes structures', field for field,
     values past fp32 and non-numbers included."""
