@@ -475,7 +475,7 @@ __global__ __launch_bounds__(256) void router_top8_kernel(const float* __restric
 // weights there (sixteen waves against eight with two tiles each: 64.1 / 65.9
 // us at 8192 tokens, 58.3 / 63.1 at 5000, bf16 46.6 / 51.4 at 8192).
 constexpr int kRtSlab = 8;          // groups per slab
-constexpr int kRtBlockWaves = 16;
+constexpr int kRtBlockWaves = 16;   // a token and a tile of 16 experts each
 
 template <int SB_DT, int X_DT>
 __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel(
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     const void* __restrict__ x, float* __restrict__ logits, int32_t* __restrict__ indices,
     float* __restrict__ scores, int experts, int cols, int batch) {
     constexpr int TERMS = rt_terms<X_DT>, XB = X_DT == 1 ? 2 : 4;                   // operands and bytes of an x
-    constexpr int NW = kRtBlockWaves, RE = 256, TW = 16 / NW, XL = XB;              // TW tiles of 16 experts per wave
+    constexpr int NW = kRtBlockWaves, RE = 16 * NW, XL = XB;
     constexpr int SBT = RE * kRtSlab / (64 * NW);                                   // scale entries per thread and slab
     constexpr int XS = 16 * 512;                                                    // values of a slab
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -493,22 +493,19 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
 
     __shared__ __attribute__((aligned(16))) uint16_t xs[2][TERMS][XS];
     __shared__ __attribute__((aligned(16))) float sbl[2][kRtSlab * (RE + 2) * 2];
-    __shared__ __attribute__((aligned(16))) uint32_t wl[NW][TW][256];   // per wave: a tile's 16 rows x 64 bytes
+    __shared__ __attribute__((aligned(16))) uint32_t wl[NW][256];   // per wave: a tile's 16 rows x 64 bytes
     __shared__ float xf[2][kRtSlab][16];   // sum of (group, token)
     __shared__ unsigned redo_s;   // bit per token: redone on the vector units
     bool redo = false;
     if (t == 0) redo_s = 0;
 
     // this thread's x quads and scale entries of a slab, and this wave's
-    // weights of it: lane (row n, kb) bytes 16 kb .. +15 of each group
-    u32x4_t xr[XL], wr[kRtSlab][TW];
+    // weights of it: lane l the 16 bytes l % 4 of row l / 4 of each group
+    u32x4_t xr[XL], wr[kRtSlab];
     float sv[SBT], bv[SBT];
     // the first eight waves' threads hold a slab's 128 (token, group) quads
     const bool stager = __builtin_amdgcn_readfirstlane(wave) < 8;   // wave-uniform
-    const uint32_t* wrow[TW];
-#pragma unroll
-    for (int i = 0; i < TW; ++i)
-        wrow[i] = w + static_cast<size_t>(min(16 * (TW * wave + i) + (lane >> 2), experts - 1)) * (cols / 4) + 4 * (lane & 3);
+    const uint32_t* const wrow = w + static_cast<size_t>(min(16 * wave + (lane >> 2), experts - 1)) * (cols / 4) + 4 * (lane & 3);
     auto fetch_x = [&](int sl) {
         if (!stager) return;
         const int q = t >> 2, tok = q >> 3, g = min(kRtSlab * sl + (q & 7), G - 1);
@@ -527,9 +524,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
         }
     };
     auto fetch_w = [&](int sl, int gl) {
-#pragma unroll
-        for (int i = 0; i < TW; ++i)
-            wr[gl][i] = *reinterpret_cast<const u32x4_t*>(wrow[i] + 16 * min(kRtSlab * sl + gl, G - 1));
+        wr[gl] = *reinterpret_cast<const u32x4_t*>(wrow + 16 * min(kRtSlab * sl + gl, G - 1));
     };
     // the fetched slab into LDS buffer buf (groups past the last get zero scales)
     auto stage = [&](int sl, int buf) {
@@ -557,14 +552,10 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     // (a clobber after each slab's requests: otherwise the compiler moves the
     // loads to the top of the iteration that uses them)
     asm volatile("" ::: "memory");
-    f32x4_t tot[TW];
-#pragma unroll
-    for (int i = 0; i < TW; ++i) tot[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    f32x4_t tot = f32x4_t{0.f, 0.f, 0.f, 0.f};   // lane: token n, experts 16 wave + 4 kb .. +3
     for (int sl = 0; sl < NS; ++sl) {
         const int buf = sl & 1;
-        f32x4_t acc[TW];   // the slab's own sums: shorter fp32 chains
-#pragma unroll
-        for (int i = 0; i < TW; ++i) acc[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};   // the slab's own sums: shorter fp32 chains
         stage(sl, buf);
         __syncthreads();
         // the next slab (the last again at the end: no branch around loads)
@@ -581,27 +572,19 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
 #pragma unroll
                 for (int k = 0; k < TERMS; ++k) xv[k][ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][k][o]);
             }
-#pragma unroll
-            for (int i = 0; i < TW; ++i) {
-                const f32x4_t P = rt_products<TERMS>(rt_tile_turn(wl[wave][i], wr[gl][i], lane), xv);
-                rt_accumulate(acc[i], P, sum,
-                              reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 16 * (TW * wave + i) + 4 * kb) * 2]));
-            }
+            const f32x4_t P = rt_products<TERMS>(rt_tile_turn(wl[wave], wr[gl], lane), xv);
+            rt_accumulate(acc, P, sum, reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 16 * wave + 4 * kb) * 2]));
             fetch_w(nx, gl);
         }
-#pragma unroll
-        for (int i = 0; i < TW; ++i) tot[i] += acc[i];
+        tot += acc;
         asm volatile("" ::: "memory");
     }
-    // lane: token n, experts 32 wave + 16 i + 4 kb .. +3
     // every expert of the 16 tokens is here: logits through LDS (the staging
     // buffers are idle once every wave is past its last slab)
     if (redo) atomicOr(&redo_s, 1u << (t >> 5));   // the token of quad t / 4
     __syncthreads();
     float* lg = reinterpret_cast<float*>(xs);   // [16][RE + 4]
-#pragma unroll
-    for (int i = 0; i < TW; ++i)
-        *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 16 * (TW * wave + i) + 4 * kb]) = tot[i];
+    *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 16 * wave + 4 * kb]) = tot;
     __syncthreads();
     if (const unsigned rd = redo_s; rd != 0) {   // workgroup-uniform
         for (int tok = 0; tok < min(16, batch - M0); ++tok) {
@@ -613,12 +596,10 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
         }
         __syncthreads();
     }
-    for (int tok = wave; tok < 16; tok += NW) {
-        const int m = M0 + tok;
-        if (m >= batch) break;
-        for (int e = lane; e < experts; e += 64) logits[static_cast<size_t>(m) * experts + e] = lg[tok * (RE + 4) + e];
-        router_top8(lg + tok * (RE + 4), indices, scores, m, experts, lane);
-    }
+    const int m = M0 + wave;
+    if (m >= batch) return;   // wave-uniform
+    for (int e = lane; e < experts; e += 64) logits[static_cast<size_t>(m) * experts + e] = lg[wave * (RE + 4) + e];
+    router_top8(lg + wave * (RE + 4), indices, scores, m, experts, lane);
 }
 
 // Q8 dequant test hook: one word (4 bytes) per thread -> 4 floats.
@@ -695,8 +676,8 @@ hipError_t launch_router_top8(qff_ctx* ctx, hipStream_t stream, const uint32_t* 
     if (vec) {                                                  \
         if (batch == 1) {                                       \
             if (k2) QFF_RV(S, X, 2, 1); else QFF_RV(S, X, 1, 1); \
-        } else {                                                \
-            if (k2) QFF_RV(S, X, 2, 4); else QFF_RV(S, X, 1, 4); \
+        } else { /* bf16 x */                                   \
+            if (k2) QFF_RV(S, 1, 2, 4); else QFF_RV(S, 1, 1, 4); \
         }                                                       \
     } else if (tiles(1) * nb <= cu) {                           \
         QFF_RM(S, X, 1, 16);                                    \
