@@ -180,33 +180,25 @@ __device__ __forceinline__ void rt_bytes_to_bf16(uint32_t w, uint32_t& lo, uint3
     hi = __builtin_amdgcn_perm(f[3], f[2], 0x07060302u);
 }
 
-// Tokens with an infinity or values near fp32's largest have their logits from
-// rt_vector_logit: an infinity leaves no terms (inf - inf), and q - 128 can
-// pass fp32's range where q, with the other sign or zero, does not.
-constexpr float kRtRange = 0x1p96f;
-
 // One group (64 columns) of one token, held by the four lanes j of a quad (fp32:
 // columns 16 i + 4 j .. +3 in piece i; bf16: 32 i + 8 j .. +7), as bf16
 // operands: a bf16 x as it is, an fp32 x as the three terms that cutting 8
 // significant bits off at a time leaves, hi + mid + lo == x with every bit (of
 // |x| >= 2^-110: below that the last term meets bf16's smallest step, 2^-133).
 // Term k goes to xo[k], LDS rows [token][row] at 16-byte pieces p0 + c,
-// swizzled by the token. Returns the sum of x; redo becomes true where the
-// lane has an |x| of kRtRange or more (a NaN makes every logit NaN either way).
+// swizzled by the token. Returns the sum of x.
 template <int X_DT, int XL>
 __device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* const (&xo)[rt_terms<X_DT>], int row,
-                                            int tok, int p0, int j, bool& redo) {
+                                            int tok, int p0, int j) {
     const int sw = tok & (row / 8 - 1) & 15;
-    float sum = 0.0f, mx = 0.0f;
+    float sum = 0.0f;
     if constexpr (X_DT == 1) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
-                const float v0 = __uint_as_float(xr[i][c] << 16), v1 = __uint_as_float(xr[i][c] & 0xffff0000u);
-                sum += v0;
-                sum += v1;
-                mx = fmaxf(fmaxf(mx, fabsf(v0)), fabsf(v1));
+                sum += __uint_as_float(xr[i][c] << 16);
+                sum += __uint_as_float(xr[i][c] & 0xffff0000u);
             }
             *reinterpret_cast<u32x4_t*>(xo[0] + tok * row + 8 * ((p0 + 4 * i + j) ^ sw)) = xr[i];
         }
@@ -218,7 +210,6 @@ __device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* c
             for (int c = 0; c < 4; ++c) {
                 const float v = __uint_as_float(xr[i][c]);
                 sum += v;
-                mx = fmaxf(mx, fabsf(v));
                 f[0][c] = xr[i][c];
                 const float r1 = v - __uint_as_float(f[0][c] & 0xffff0000u);
                 f[1][c] = __float_as_uint(r1);
@@ -231,7 +222,6 @@ __device__ __forceinline__ float rt_stage_x(const u32x4_t (&xr)[XL], uint16_t* c
                                                                  __builtin_amdgcn_perm(f[k][3], f[k][2], 0x07060302u)};
         }
     }
-    redo |= mx >= kRtRange;
     return group_sum<4>(sum);
 }
 
@@ -254,6 +244,22 @@ __device__ __forceinline__ f32x4_t rt_products(u32x4_t wd, const u32x4_t (&xo)[T
         P = mfma_16x16x32_bf16(a[1], xo[k][1], P);
     }
     return P;
+}
+
+// Logits that the products leave infinite or NaN, from the vector form: an
+// infinite x has no terms (inf - inf), and (q - 128) x can pass fp32's range
+// where q x does not. Lane l holds logit v of (token m, expert e), if ok.
+template <int SB_DT, int X_DT>
+__device__ __forceinline__ float rt_finite_or_vector(float v, bool ok, int m, int e, const uint32_t* w,
+                                                     const uint16_t* scales, const uint16_t* biases, const void* x,
+                                                     int cols, int lane) {
+    for (uint64_t bad = __ballot(ok && !(fabsf(v) <= 3.4028235e38f)); bad != 0; bad &= bad - 1) {   // wave-uniform
+        const int src = __builtin_ctzll(bad);
+        const float r = rt_vector_logit<SB_DT, X_DT>(w, scales, biases, x, cols, __builtin_amdgcn_readlane(m, src),
+                                                     __builtin_amdgcn_readlane(e, src), lane);
+        if (lane == src) v = r;
+    }
+    return v;
 }
 
 // acc += s P + (b + 128 s) sum(x) for the lane's four experts, sb their (s, b + 128 s)
@@ -300,9 +306,6 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
     __shared__ __attribute__((aligned(16))) uint32_t wl[NW][256];
     __shared__ __attribute__((aligned(16))) uint16_t xl[NW][TERMS][16 * 64];
     __shared__ float xf[NW][16];
-    __shared__ unsigned redo_s;   // bit per token: redone on the vector units
-    bool redo = false;
-    if (t == 0) redo_s = 0;
 
     const char* xrow = static_cast<const char*>(x) +
                        static_cast<size_t>(min(M0 + (lane >> 2), batch - 1)) * cols * XB + 16 * (lane & 3);
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
         uint16_t* xo[TERMS];
 #pragma unroll
         for (int k = 0; k < TERMS; ++k) xo[k] = xl[wave][k];
-        const float xs = rt_stage_x<X_DT>(xr[s], xo, 64, lane >> 2, 0, lane & 3, redo);
+        const float xs = rt_stage_x<X_DT>(xr[s], xo, 64, lane >> 2, 0, lane & 3);
         if ((lane & 3) == 0) xf[wave][lane >> 2] = xs;
         __builtin_amdgcn_wave_barrier();
         const float sum = xf[wave][n];
@@ -372,26 +375,18 @@ __global__ __launch_bounds__(64 * NW) void router_logits_mfma_kernel(const uint3
         if (g + NW < G) step(1, g + NW);
         if (g + 3 * NW < G) fetch(1, g + 3 * NW);
     }
-    if (redo) atomicOr(&redo_s, 1u << (lane >> 2));
     __syncthreads();   // the scales are consumed; their bytes take the partial sums
 #pragma unroll
     for (int i = 0; i < NT; ++i) *reinterpret_cast<f32x4_t*>(&lds[wave * RE * 16 + (i * 64 + lane) * 4]) = acc[i];
     __syncthreads();
-    const unsigned rd = redo_s;
-    for (int o = t; o < RE * 16; o += 64 * NW) {
+    for (int o = t; o < RE * 16; o += 64 * NW) {   // wave-uniform
         float v = lds[o];
 #pragma unroll
         for (int ww = 1; ww < NW; ++ww) v += lds[ww * RE * 16 + o];
         const int l = (o >> 2) & 63, e = E0 + 16 * (o >> 8) + 4 * (l >> 4) + (o & 3), m = M0 + (l & 15);
-        if (m < batch && e < experts && !(rd >> (l & 15) & 1)) logits[static_cast<size_t>(m) * experts + e] = v;
-    }
-    if (rd == 0) return;   // workgroup-uniform
-    for (int tok = 0; tok < min(16, batch - M0); ++tok) {
-        if (!(rd >> tok & 1)) continue;
-        for (int e = E0 + wave; e < min(E0 + RE, experts); e += NW) {
-            const float v = rt_vector_logit<SB_DT, X_DT>(w, scales, biases, x, cols, M0 + tok, e, lane);
-            if (lane == 0) logits[static_cast<size_t>(M0 + tok) * experts + e] = v;
-        }
+        const bool ok = m < batch && e < experts;
+        v = rt_finite_or_vector<SB_DT, X_DT>(v, ok, m, e, w, scales, biases, x, cols, lane);
+        if (ok) logits[static_cast<size_t>(m) * experts + e] = v;
     }
 }
 
@@ -495,9 +490,6 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     __shared__ __attribute__((aligned(16))) float sbl[2][kRtSlab * (RE + 2) * 2];
     __shared__ __attribute__((aligned(16))) uint32_t wl[NW][256];   // per wave: a tile's 16 rows x 64 bytes
     __shared__ float xf[2][kRtSlab][16];   // sum of (group, token)
-    __shared__ unsigned redo_s;   // bit per token: redone on the vector units
-    bool redo = false;
-    if (t == 0) redo_s = 0;
 
     // this thread's x quads and scale entries of a slab, and this wave's
     // weights of it: lane l the 16 bytes l % 4 of row l / 4 of each group
@@ -540,7 +532,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
             uint16_t* xo[TERMS];
 #pragma unroll
             for (int k = 0; k < TERMS; ++k) xo[k] = xs[buf][k];
-            const float sum = rt_stage_x<X_DT>(xr, xo, 512, tok, 8 * gl, j, redo);
+            const float sum = rt_stage_x<X_DT>(xr, xo, 512, tok, 8 * gl, j);
             if (j == 0) xf[buf][gl][tok] = sum;
         }
     };
@@ -581,25 +573,21 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     }
     // every expert of the 16 tokens is here: logits through LDS (the staging
     // buffers are idle once every wave is past its last slab)
-    if (redo) atomicOr(&redo_s, 1u << (t >> 5));   // the token of quad t / 4
     __syncthreads();
     float* lg = reinterpret_cast<float*>(xs);   // [16][RE + 4]
     *reinterpret_cast<f32x4_t*>(&lg[n * (RE + 4) + 16 * wave + 4 * kb]) = tot;
     __syncthreads();
-    if (const unsigned rd = redo_s; rd != 0) {   // workgroup-uniform
-        for (int tok = 0; tok < min(16, batch - M0); ++tok) {
-            if (!(rd >> tok & 1)) continue;
-            for (int e = wave; e < experts; e += NW) {
-                const float v = rt_vector_logit<SB_DT, X_DT>(w, scales, biases, x, cols, M0 + tok, e, lane);
-                if (lane == 0) lg[tok * (RE + 4) + e] = v;
-            }
-        }
-        __syncthreads();
-    }
     const int m = M0 + wave;
     if (m >= batch) return;   // wave-uniform
-    for (int e = lane; e < experts; e += 64) logits[static_cast<size_t>(m) * experts + e] = lg[wave * (RE + 4) + e];
-    router_top8(lg + wave * (RE + 4), indices, scores, m, experts, lane);
+    lg += wave * (RE + 4);
+    for (int e0 = 0; e0 < experts; e0 += 64) {
+        const int e = e0 + lane;
+        const bool ok = e < experts;
+        const float v = rt_finite_or_vector<SB_DT, X_DT>(lg[e], ok, m, e, w, scales, biases, x, cols, lane);
+        if (ok) logits[static_cast<size_t>(m) * experts + e] = lg[e] = v;
+    }
+    __builtin_amdgcn_wave_barrier();
+    router_top8(lg, indices, scores, m, experts, lane);
 }
 
 // Q8 dequant test hook: one word (4 bytes) per thread -> 4 floats.
