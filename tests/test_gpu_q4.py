@@ -364,6 +364,40 @@ def test_q4_many_tokens_split_tiles(hip, batch, cols, odd):
         assert _rel(got, ref) <= (1e-3 if dt == torch.float32 else 4e-3)
 
 
+@pytest.mark.parametrize("batch,cols", [(1003, 4096), (803, 3200)])
+def test_q4_many_tokens_large_split_tiles(hip, batch, cols):
+    """The 64 x 64 split tiles and the eight-token fp16 pass at ragged rows,
+    tokens and column blocks: 2048 rows with an fp32 residual in place, 100
+    with a bf16 one, 3 rows, and 64 rows with residuals that 16- and 8-byte
+    loads cannot take (one element past a boundary); bf16 scales; within 1e-3
+    of the fp64 product (fp16 operands), bf16 outputs 4e-3."""
+    import qff
+    print(f"q4 large split tiles batch={batch} cols={cols}", flush=True)
+    shapes = [(2048, "f32", False), (100, "bf16", False), (3, "f32", False), (64, "f32", True), (64, "bf16", True)]
+    ws = [synth.q4_weight(r, cols, seed=10 * i + r, sb_dtype="bf16") for i, (r, _, _) in enumerate(shapes)]
+    rng = np.random.default_rng(batch)
+    x = rng.standard_normal((batch, cols)).astype(np.float32)
+    res = [O.round_bf16((30 * rng.standard_normal((batch, r))).astype(np.float32)) for r, _, _ in shapes]
+
+    def gpu(v, dt, odd):
+        t = f32_tensor(v) if dt == "f32" else bf16_tensor(O.f32_to_bf16(v))
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape) if odd else t
+
+    rt = [gpu(v, dt, odd) for v, (_, dt, odd) in zip(res, shapes)]
+    ys = [rt[0]] + [torch.empty(t.shape, dtype=t.dtype, device=DEV) for t in rt[1:]]
+    ctx = qff.Context(max_batch=1, max_ctx=64, max_prefill_tokens=64)
+    outs = qff.q4_matmul_parts(ctx, [_w_gpu(*w, "bf16") for w in ws], f32_tensor(x), outs=ys, residuals=rt)
+    torch.cuda.synchronize()
+    for (r, dt, odd), w, got, v in zip(shapes, ws, outs, res):
+        ref = x.astype(np.float64) @ O.q4_dequant(*w, O.BF16).astype(np.float64).T
+        if dt == "f32":
+            assert _rel(to_np(got).astype(np.float64) - v, ref) <= 1e-3, (r, dt, odd)
+        else:
+            assert _rel(to_np(got).astype(np.float64), ref + v) <= 4e-3, (r, dt, odd)
+            # the residual and the product each, where rounding to bf16 is small beside both
+            assert _rel(to_np(got).astype(np.float64) - v, ref) <= 2e-2, (r, dt, odd)
+
+
 @pytest.mark.parametrize("batch,cols", [(40, 4096), (70, 2048), (300, 2048)])
 def test_q4_part_does_not_depend_on_the_parts_beside_it(hip, batch, cols):
     """A part's outputs bit for bit the same alone and beside others: one with
