@@ -287,8 +287,11 @@ static_assert(2 * kC * 65 * 4 <= 2 * kTile128, "T must fit the Q region");
 //       substitution (one wave each), the off-diagonal blocks by halves on
 //       fp32 MFMAs;
 //   T blocks out.
-// Global loads are issued before the stores of the same unit (vmcnt counts
-// stores too on gfx950, so a load consumed after stores would wait for them).
+// vmcnt counts stores too on gfx950, so a load waits for the stores issued
+// before it. Waves 0-3 issue the next unit's loads ahead of the K image, Q and T
+// stores. Waves 4-7 issue theirs after all of their stores but T's: they wait
+// for those in the next unit's first phase, a phase of inversion later, which
+// costs less than 60 loads in the phase of their P blocks, the longer one.
 constexpr int kLocalThreads = 512;
 
 template <int IN_DT>
@@ -316,8 +319,9 @@ __global__ __launch_bounds__(kLocalThreads) void dn_chunk_local_kernel(
     fetch_unit<IN_DT>(in, u, T, qkv, a, b, a_log, dt_bias, conv_w, threadIdx.x >> 6, threadIdx.x & 63);
     if (threadIdx.x == 0) s_next = 2 * grid + static_cast<int>(atomicAdd(sched, 1u));
     // Wait here for the first unit's loads: the loop's own waits then only
-    // count the operations of the previous iteration, which issues stores
-    // after its prefetch, so consuming the prefetch does not wait for them.
+    // count the operations of the previous iteration, where the T stores (on
+    // waves 0-3 the K image's and Q's too) follow the prefetch, so that
+    // consuming it does not wait for them.
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
