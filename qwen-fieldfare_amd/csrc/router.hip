@@ -29,8 +29,8 @@
 //       so the logits are closer to the fp64 product than the vector form's
 //       (2000 tokens of fp32 x, 2-norm: 0.92e-7 against 2.5e-7; bf16 x 0.81e-7
 //       against 0.91e-7). x as an fp16 hi + lo pair (22 bits) took two thirds
-//       of the products and 1.05e-7: 25.6 us at 2000 tokens either way, 54.6
-//       against 64 at 8192. NW waves split K.
+//       of the products and 1.05e-7: 25.6 us at 2000 tokens either way, 54.4
+//       against 58.5 at 8192. NW waves split K.
 //       What bounded the first form of it, at 25-30 us a block, was the
 //       operand order itself: a lane per matrix row makes a 16-byte load
 //       touch 64 different lines (38 B/ns per CU from L2 against 125-148
@@ -465,11 +465,13 @@ __global__ __launch_bounds__(256) void router_top8_kernel(const float* __restric
 // w experts 16 w .. 16 w + 15, one MFMA tile over all of K) and ranks its
 // tokens itself, one per wave. Each slab of 512 columns of x is converted
 // once per workgroup (thread quads, rt_stage_x) into LDS; the weights are
-// requested a slab ahead into registers. What seems to bound it is LDS: every
-// wave reads the slab's x (3 MB a block in all, 1 MB of bf16) and turns its
-// weights there (sixteen waves against eight with two tiles each: 64.1 / 65.9
-// us at 8192 tokens, 58.3 / 63.1 at 5000, bf16 46.6 / 51.4 at 8192).
+// requested four groups ahead into registers (a slab ahead ten registers
+// spill: 21 MB of scratch writes, 64 against 58.5 us at 8192 tokens). What
+// seems to bound it is LDS: every wave reads the slab's x (3 MB a block in all,
+// 1 MB of bf16) and turns its weights there. Eight waves with two tiles each:
+// 3-8 % slower than these sixteen, 10 % with bf16 x.
 constexpr int kRtSlab = 8;          // groups per slab
+constexpr int kRtAhead = 4;         // groups between a weight tile's request and its use
 constexpr int kRtBlockWaves = 16;   // a token and a tile of 16 experts each
 
 template <int SB_DT, int X_DT>
@@ -493,7 +495,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
 
     // this thread's x quads and scale entries of a slab, and this wave's
     // weights of it: lane l the 16 bytes l % 4 of row l / 4 of each group
-    u32x4_t xr[XL], wr[kRtSlab];
+    u32x4_t xr[XL], wr[kRtAhead];
     float sv[SBT], bv[SBT];
     // the first eight waves' threads hold a slab's 128 (token, group) quads
     const bool stager = __builtin_amdgcn_readfirstlane(wave) < 8;   // wave-uniform
@@ -515,9 +517,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
             bv[k] = elem<SB_DT>::load(biases, gi);
         }
     };
-    auto fetch_w = [&](int sl, int gl) {
-        wr[gl] = *reinterpret_cast<const u32x4_t*>(wrow + 16 * min(kRtSlab * sl + gl, G - 1));
-    };
+    auto fetch_w = [&](int g) { wr[g & (kRtAhead - 1)] = *reinterpret_cast<const u32x4_t*>(wrow + 16 * min(g, G - 1)); };
     // the fetched slab into LDS buffer buf (groups past the last get zero scales)
     auto stage = [&](int sl, int buf) {
 #pragma unroll
@@ -540,7 +540,7 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
     fetch_x(0);
     fetch_sb(0);
 #pragma unroll
-    for (int gl = 0; gl < kRtSlab; ++gl) fetch_w(0, gl);
+    for (int g = 0; g < kRtAhead; ++g) fetch_w(g);
     // (a clobber after each slab's requests: otherwise the compiler moves the
     // loads to the top of the iteration that uses them)
     asm volatile("" ::: "memory");
@@ -564,9 +564,9 @@ __global__ __launch_bounds__(64 * kRtBlockWaves) void router_logits_block_kernel
 #pragma unroll
                 for (int k = 0; k < TERMS; ++k) xv[k][ks] = *reinterpret_cast<const u32x4_t*>(&xs[buf][k][o]);
             }
-            const f32x4_t P = rt_products<TERMS>(rt_tile_turn(wl[wave], wr[gl], lane), xv);
+            const f32x4_t P = rt_products<TERMS>(rt_tile_turn(wl[wave], wr[gl % kRtAhead], lane), xv);
             rt_accumulate(acc, P, sum, reinterpret_cast<const f32x4_t*>(&sbl[buf][(gl * (RE + 2) + 16 * wave + 4 * kb) * 2]));
-            fetch_w(nx, gl);
+            fetch_w(kRtSlab * sl + gl + kRtAhead);
         }
         tot += acc;
         asm volatile("" ::: "memory");
@@ -632,7 +632,7 @@ hipError_t launch_router_top8(qff_ctx* ctx, hipStream_t stream, const uint32_t* 
     //   MFMA, 1 tile    161 / 85.3 / 57.0 / 46.4 / 17.1 / 11.8 / 11.0  103 / 55.5 / 37.9 / 31.3 / 12.8 / 10.2 / 9.5
     //   MFMA, 2 tiles   120 / 67.1 / 46.6 / 37.9 / 14.2 / 12.9 / 12.4   65 / 36.6 / 26.4 / 22.5 / 11.4 / 11.1 / 10.7
     //   MFMA, 4 tiles    82 / 43.9 / 35.1 / 25.2 / 17.3 / 17.3 / 17.0   58 / 33.8 / 25.6 / 20.4 / 15.4 / 15.4 / 14.8
-    //   whole blocks     64 / 33.7 / 30.4 / 30.3 / 29.1 / 28.9 / 27.7   47 / 24.6 / 23.1 / 22.8 / 23.1 / 23.0 / 21.8
+    //   whole blocks   58.5 / 31.1 / 28.9 / 30.3 / 29.1 / 28.9 / 27.7   45 / 24.2 / 23.0 / 22.8 / 23.1 / 23.0 / 21.8
     // so the tiles per workgroup grow once the grid covers the chip, and whole
     // blocks take over where they do so themselves.
     const int nb = (batch + 15) / 16, cu = ctx->num_cu;
