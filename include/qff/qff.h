@@ -192,9 +192,9 @@ int qff_q8_dequant(qff_ctx* ctx, qff_stream_t stream, const uint32_t* w,
  * factored form scale * sum(q x) + bias * sum(x) per group (several tokens:
  * over q - 128 with the bias adjusted, an fp32 x as three bf16 terms that hold
  * every bit of |x| >= 2^-110; so a token's logits can differ in the last bits
- * between batch sizes); then per token the eight largest logits in descending order (equal logits: lower expert
- * index first) into indices [batch, 8], and their routing weights into
- * scores [batch, 8]: softmax over all `experts` logits shifted by the
+ * between batch sizes); then per token the eight largest logits in
+ * descending order (equal logits: lower expert index first) into indices
+ * [batch, 8], and their routing weights into scores [batch, 8]: softmax over all `experts` logits shifted by the
  * largest, the eight probabilities divided by their sum. x [batch, cols] of
  * x_dtype (F32 or BF16), logits [batch, experts] fp32 (written). Replaces
  * qwen_router_q8_logits_simd_f32 + qwen_router_top8_logits_f32

@@ -466,10 +466,11 @@ __global__ __launch_bounds__(256) void router_top8_kernel(const float* __restric
 // tokens itself, one per wave. Each slab of 512 columns of x is converted
 // once per workgroup (thread quads, rt_stage_x) into LDS; the weights are
 // requested four groups ahead into registers (a slab ahead ten registers
-// spill: 21 MB of scratch writes, 64 against 58.5 us at 8192 tokens). What
-// seems to bound it is LDS: every wave reads the slab's x (3 MB a block in all,
-// 1 MB of bf16) and turns its weights there. Eight waves with two tiles each:
-// 3-8 % slower than these sixteen, 10 % with bf16 x.
+// spill: 21 MB of scratch writes, 64 against 58.5 us at 8192 tokens). LDS is
+// active half of the time at 8192 tokens, a fifth of that on bank conflicts, and
+// the matrix cores 16 %: every wave reads the slab's x (3 MB a block in all, 1
+// MB of bf16) and turns its weights there. Eight waves with two tiles each: 3-8
+// % slower than these sixteen, 10 % with bf16 x.
 constexpr int kRtSlab = 8;          // groups per slab
 constexpr int kRtAhead = 4;         // groups between a weight tile's request and its use
 constexpr int kRtBlockWaves = 16;   // a token and a tile of 16 experts each
