@@ -1084,7 +1084,9 @@ __device__ __forceinline__ u32x4_t q4_to_f16_scaled(uint32_t w, uint32_t sb, uin
     return r;
 }
 
-template <int SB_DT>
+// RES: some part has a residual (as a run-time branch the epilogue of products
+// without one took 2-3 us more).
+template <int SB_DT, bool RES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q4_gemm_kernel(
     Q4Parts parts, const uint16_t* __restrict__ x16, const float* __restrict__ fm, int cols, int batch) {
     // the part of this workgroup's row tile (parts' tiles are consecutive in x)
@@ -1094,7 +1096,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     const uint16_t* __restrict__ scales = parts.s[pp];
     const uint16_t* __restrict__ biases = parts.b[pp];
     void* __restrict__ y = parts.y[pp];
-    const void* __restrict__ res = parts.res[pp];
+    const void* __restrict__ res = RES ? parts.res[pp] : nullptr;
     const int rows = parts.rows[pp];
     const bool ybf = parts.ybf16[pp];
     const int G = cols / 64;
@@ -1199,12 +1201,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     }
     if (g < G) step(0, g);
 
-    // lane: token 32 mt + r, rows 64 wave + 32 rt + 8 j + 4 h .. +3 (adjacent in y)
+    // lane: token 32 mt + r, rows 64 wave + 32 rt + 8 j + 4 h .. +3 (adjacent in
+    // y); a token's residuals all requested before the first is used (indices
+    // clamped; one at a time they cost 15 us at 2048 x 4096 x 4096 tokens)
+    const bool rvec = res != nullptr && (rows & 3) == 0 && (reinterpret_cast<uintptr_t>(res) & 15) == 0;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
         const int m = M0 + 32 * mt + r;
         if (m >= batch) continue;
         const float f = fm[m];
+        f32x4_t rv[2][4];
+        if (rvec) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const int rr = min(R0 + 64 * wave + 32 * (i >> 2) + 8 * (i & 3) + 4 * h, rows - 4);
+                const size_t o = static_cast<size_t>(m) * rows + rr;
+                if (ybf) {
+                    const u32x2_t u = *reinterpret_cast<const u32x2_t*>(static_cast<const uint16_t*>(res) + o);
+                    rv[i >> 2][i & 3] = f32x4_t{__uint_as_float(u[0] << 16), __uint_as_float(u[0] & 0xffff0000u),
+                                                __uint_as_float(u[1] << 16), __uint_as_float(u[1] & 0xffff0000u)};
+                } else {
+                    rv[i >> 2][i & 3] = *reinterpret_cast<const f32x4_t*>(static_cast<const float*>(res) + o);
+                }
+            }
+        }
 #pragma unroll
         for (int rt = 0; rt < 2; ++rt)
 #pragma unroll
@@ -1216,7 +1236,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     v[i] *= f;
-                    if (res && rr + i < rows) v[i] += ybf ? elem<1>::load(res, o + i) : elem<0>::load(res, o + i);
+                    if (rvec) v[i] += rv[rt][j][i];
+                    else if (res && rr + i < rows) v[i] += ybf ? elem<1>::load(res, o + i) : elem<0>::load(res, o + i);
                 }
                 if (rr + 3 < rows && (rows & 3) == 0) {
                     if (ybf)
@@ -1491,8 +1512,10 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
                                 int cols, int batch) {
     const int G = cols / 64;
     const int lds = G * kQ4GemmRows * 4;   // packed (s, b) of the row tile
-    QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<1>>(lds)));
-    QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<2>>(lds)));
+    QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<1, false>>(lds)));
+    QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<1, true>>(lds)));
+    QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<2, false>>(lds)));
+    QFF_CHECK_HIP_RET((q4_allow_lds<q4_gemm_kernel<2, true>>(lds)));
     // Which kernel: part by part, and K always split in four, so that a part's
     // sums do not depend on the rows beside it (the split tiles read scales
     // and biases two groups at a time: an even number of groups,
@@ -1579,10 +1602,14 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
         q4_gemm_split_kernel<2, RT, MT, WK, D><<<grid, 64 * WK, 0, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb, pm)
             if (!split) {
                 grid = pack_grid(kQ4GemmRows, kQ4GemmToks, P);
-                if (sb_dtype == QFF_BF16)
-                    q4_gemm_kernel<1><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
-                else
-                    q4_gemm_kernel<2><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb);
+                const bool res = std::any_of(sl, sl + n, [](const qff_q4_part& q) { return q.residual != nullptr; });
+#define QFF_LARGE(S, R) q4_gemm_kernel<S, R><<<grid, 256, lds, stream>>>(P, ctx->q4_x16, ctx->q4_fm, cols, mb)
+                if (sb_dtype == QFF_BF16) {
+                    if (res) QFF_LARGE(1, true); else QFF_LARGE(1, false);
+                } else {
+                    if (res) QFF_LARGE(2, true); else QFF_LARGE(2, false);
+                }
+#undef QFF_LARGE
             } else if (count(grid = pack_grid(32, 32, P)) <= cu) {
                 QFF_SPLIT(1, 1, 4, 2);
             } else if (count(grid = pack_grid(32, 64, P)) <= cu) {

@@ -364,15 +364,15 @@ def test_q4_many_tokens_split_tiles(hip, batch, cols, odd):
         assert _rel(got, ref) <= (1e-3 if dt == torch.float32 else 4e-3)
 
 
-@pytest.mark.parametrize("batch,cols", [(1003, 4096), (803, 3200)])
-def test_q4_many_tokens_large_split_tiles(hip, batch, cols):
-    """The 64 x 64 split tiles and the eight-token fp16 pass at ragged rows,
-    tokens and column blocks: 2048 rows with an fp32 residual in place, 100
+@pytest.mark.parametrize("batch,cols", [(1003, 4096), (803, 3200), (460, 2048)])
+def test_q4_many_tokens_ragged_tiles_with_residuals(hip, batch, cols):
+    """The 64 x 64 split tiles with the eight-token fp16 pass, and the large
+    tile, at ragged rows, tokens and column blocks: 2048 rows with an fp32 residual in place, 100
     with a bf16 one, 3 rows, and 64 rows with residuals that 16- and 8-byte
     loads cannot take (one element past a boundary); bf16 scales; within 1e-3
     of the fp64 product (fp16 operands), bf16 outputs 4e-3."""
     import qff
-    print(f"q4 large split tiles batch={batch} cols={cols}", flush=True)
+    print(f"q4 ragged tiles with residuals batch={batch} cols={cols}", flush=True)
     shapes = [(2048, "f32", False), (100, "bf16", False), (3, "f32", False), (64, "f32", True), (64, "bf16", True)]
     ws = [synth.q4_weight(r, cols, seed=10 * i + r, sb_dtype="bf16") for i, (r, _, _) in enumerate(shapes)]
     rng = np.random.default_rng(batch)
