@@ -1534,27 +1534,31 @@ static hipError_t q4_gemm_parts(qff_ctx* ctx, hipStream_t stream, const qff_q4_p
     // Up to 2048 columns the widest in-projection sets the line at 448 tokens;
     // above, 4096 tokens is as far as split tiles were tried (2048 rows would
     // still gain beyond). Below these lines a part of more than 64 tokens
-    // takes the large tile where its own tiles fill the chip: large / split at
-    //   32768 x 2048, 200 / 448 tokens       54 / 58      83 / 99
-    //   151936 x 2048, 64 / 128 / 448       104 / 68     116 / 128    342 / 435
-    //   8192 x 3072, 700 / 1000 / 2000       68 / 59      76 / 77     120 / 145
-    //   2048 x 3072, 2000 / 3000 / 4096      69 / 47      73 / 65      83 / 84
-    // Above 3072 columns, where the scales of all of K in LDS leave one large
-    // workgroup a CU, it takes whole rounds of them (a large tile of a full
-    // round costs as much as 7.4 of the eight split tiles in it):
-    //   8192 x 4096, 700 / 1000 / 4096       86 / 74      97 / 97     362 / 375
-    //   12352 x 4096, 512 / 700 / 2000       89 / 84     167 / 107    347 / 279
-    //   32768 x 4096, 448 / 512 / 2000      177 / 167    180 / 189    694 / 745
+    // takes the large tile where its own large tiles fill the chip. us large /
+    // split, then with an fp32 residual, which costs the large tile more (the
+    // kernel must not follow from it: the sums would):
+    //   32768 x 2048, 129 / 200 / 448 tokens    51 / 46   53 / 56   83 / 99     - 57 / 56   89 / 98
+    //   65536 x 2048, 65 / 128 / 200            48 / 55   52 / 58   79 / 108    51 / 55  58 / 59  84 / 108
+    //   8192 x 3072, 1000 / 1500 / 2000         76 / 77  106 / 110 122 / 144    79 / 77 112 / 110 128 / 144
+    // At one large tile a CU a draw but for wide parts, which seldom have a
+    // residual: others take it from one and a half. Above 3072 columns the
+    // scales of all of K in LDS leave one large workgroup a CU, so it takes whole
+    // rounds of them (a large tile of a full round costs as much as 7.4 of the
+    // eight split tiles in it), and only of wide parts:
+    //   32768 x 4096, 448 / 512 / 2000         177 / 167 179 / 193 688 / 745    - 189 / 194 742 / 762
+    //   8192 x 4096, 700 / 1024 / 4096          88 / 76   97 / 100 363 / 377    - 100 / 98 381 / 377
+    //   2048 x 4096, 3968 / 4096               105 / 104 108 / 106             110 / 104 113 / 106
     const int cu = ctx->num_cu, tb = std::min(batch, ctx->q4_xs_tokens);
     const auto takes_split = [&](const qff_q4_part& q) {
         if ((cols / 64) % 2 != 0 || batch > (cols > 2048 ? 4096 : 448) ||
             ((reinterpret_cast<uintptr_t>(q.scales) | reinterpret_cast<uintptr_t>(q.biases)) & 3) != 0)
             return false;
-        const long long large = static_cast<long long>((q.rows + kQ4GemmRows - 1ll) / kQ4GemmRows) *
-                                ((tb + kQ4GemmToks - 1) / kQ4GemmToks);
-        const long long small = (q.rows + 63ll) / 64 * ((tb + 63) / 64);
         if (tb <= 64) return true;
-        return cols <= 3072 ? large < cu : (large + cu - 1) / cu * cu * 80 > small * 11;
+        const bool wide = q.rows / 4 >= cols;
+        const long long large = (q.rows + kQ4GemmRows - 1ll) / kQ4GemmRows * ((tb + kQ4GemmToks - 1) / kQ4GemmToks);
+        const long long small = (q.rows + 63ll) / 64 * ((tb + 63) / 64);   // eight in a large tile
+        if (cols <= 3072) return 2 * large < (wide ? 2 : 3) * cu || 8 * large > 1.25 * small;
+        return !wide || 8 * ((large + cu - 1) / cu * cu) > 1.08 * small;
     };
     const int pm = (1 << 20) / std::max(G / 2, 1) + 1;   // idx / (G / 2) = idx pm >> 20, idx < 2048
     for (int m0 = 0; m0 < batch; m0 += ctx->q4_xs_tokens) {

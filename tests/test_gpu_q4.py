@@ -420,8 +420,8 @@ def test_q4_part_does_not_depend_on_the_parts_beside_it(hip, batch, cols):
         assert torch.equal(alone, both[i]), i
 
 
-@pytest.mark.parametrize("rows,cols,batch,over", [(32768, 2048, 200, 449), (32768 + 5, 2048, 130, 449),
-                                                  (8192, 3072, 1100, 4097), (32768, 4096, 512, 4097)])
+@pytest.mark.parametrize("rows,cols,batch,over", [(32768, 2048, 200, 449), (65536 + 5, 2048, 100, 449),
+                                                  (8192, 3072, 1990, 4097), (32768, 4096, 512, 4097)])
 def test_q4_wide_part_takes_the_large_tile(hip, rows, cols, batch, over):
     """A part whose own large tiles fill the chip: its outputs are bit for bit
     those of the first tokens of a batch that always takes that tile, within
